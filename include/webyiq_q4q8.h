@@ -135,7 +135,7 @@ int wq_quant_gemv(void* stream, const float* x, const float* norm_w, float eps,
                   int64_t M, int32_t mode, int8_t* xq, float* dx, int32_t* xs, float* y);
 
 /*
- * Prefill GEMM, any M >= 1 (tiles of 128 tokens).  Replaces Builder::gemm
+ * Prefill GEMM, any M >= 1 (tiles of 128 or 32 tokens).  Replaces Builder::gemm
  * (graph.rs:200-205, which binds the step's Params) and
  * gemm_q4q8.wgsl:46-121.  Same arguments and constraints as wq_gemv, plus
  * M * K and rows * K / 2 (rows = N, or 2N in WQ_MODE_SILU_MUL) below 4 GiB.
@@ -145,11 +145,11 @@ int wq_quant_gemv(void* stream, const float* x, const float* norm_w, float eps,
  * 0 .. min(params->m, M) - 1 are computed and stored, rows past them are
  * neither read beyond row M - 1 nor written, and token tiles past them end at
  * once (the reference clamps its tokens to p.m, gemm_q4q8.wgsl:69,106).
- * The int32 group sums are the GEMV's; with per-token activations (G = 128
- * or 32) the min term is summed on an f16 MFMA (exact products, fp32 sums in
- * hardware order) and per-32 activations fold one chain per output (the
- * GEMV: chains and a tree): the fp32 outputs agree with wq_gemv within
- * rel 1e-5.
+ * The int32 group sums are the GEMV's; the min term is summed on the matrix
+ * cores (exact products with per-token activations, fp32 sums in hardware
+ * order), and calls of few tokens or with per-32 activations split K between
+ * the waves of a workgroup and add the parts in one fixed order: the fp32
+ * outputs are deterministic and agree with wq_gemv within rel 1e-5.
  * workspace (device, nullable, 256-byte aligned; no counterpart in the
  * reference): when it holds at least wq_gemm_workspace_bytes(...) > 0 bytes
  * for the call's shape, the K steps of each output tile may be split between

@@ -1,0 +1,92 @@
+"""The GEMM with K split between the waves of a workgroup (gemm_wave.hip),
+against the CPU oracle at the edges of its tiles: 32 tokens x 32 or 64 rows,
+4 or 8 waves, fewer K steps than waves and step counts the waves do not share
+evenly, ragged rows and tokens, and scale, sum and dx arrays that are only
+4-byte aligned (the kernel reads their four-word pieces word by word then).
+
+fp32 outputs within rel 1e-5 (max-norm) of the oracle, the bar of the other
+GEMM tests: the int32 group sums are exact, and the fp32 sums of K / G terms
+differ from the oracle's order by a few 2^-24 relative to the largest term.
+"""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as orc
+from oracle import reference as ref
+from webyiq_amd import ops
+from conftest import rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def dev(a, shift=0):
+    """a on the GPU, its first element `shift` elements past a 256-byte boundary."""
+    t = torch.empty(a.size + 64, dtype=torch.from_numpy(a).dtype, device="cuda")
+    t = t[shift:shift + a.size].view(a.shape)
+    t.copy_(torch.from_numpy(np.ascontiguousarray(a)))
+    return t
+
+
+FORMATS = [(128, None), (32, None), (32, 32), (128, 32)]
+
+
+@pytest.mark.parametrize("G,GA", FORMATS)
+@pytest.mark.parametrize("M,K,N,mode,shift", [
+    (1, 128, 1, 0, 0),        # one step: seven waves without work
+    (33, 1152, 33, 1, 0),     # nine steps over eight waves, one token and one row past a tile
+    (31, 640, 65, 2, 1),      # gate/up pairs, five steps, unaligned arrays
+    (32, 2048, 97, 0, 3),     # unaligned arrays, narrow tiles
+    (300, 512, 2100, 0, 2),   # more than 256 tiles of 64 rows: four waves, unaligned arrays
+    (520, 384, 1025, 1, 0),   # three steps over four waves
+])
+def test_wave_gemm_edges(M, K, N, mode, shift, G, GA):
+    print(f"[case] wave gemm M={M} K={K} N={N} G={G} GA={GA} mode={mode} shift={shift}", flush=True)
+    rng = np.random.default_rng(M + K + N + mode)
+    rows = 2 * N if mode == 2 else N
+    wq, ws = ref.make_weight(rng, rows, K, G)
+    x = ref.make_activations(rng, M, K)
+    gaa = K if GA is None else GA
+    xq, dx, xs = orc.quant_act(x, GA, G)
+    y0 = rng.normal(size=(M, N)).astype(np.float32) if mode == 1 else None
+    want = orc.linear(wq, ws, K, G, xq, dx, xs, mode=mode, y=y0, GA=gaa)
+    w = ops.Q4Tensor(dev(wq.view("int32")), dev(ws.view("int32"), shift), K, G)
+    a = ops.Acts(dev(xq), dev(dx, shift), dev(xs, shift), gaa, G)
+
+    def run(m=None):
+        y = dev(y0) if mode == 1 else torch.full((M, N), float("nan"), device="cuda")
+        ops.gemm(w, a, mode=mode, y=y, params=None if m is None else ops.make_params(m=m))
+        torch.cuda.synchronize()
+        return y.cpu().numpy()
+    got = run()
+    assert rel_err(got, want) < 1e-5
+    m = (M + 1) // 2  # device Params below the capacity: the same rows, the others untouched
+    part = run(m)
+    assert np.array_equal(part[:m].view(np.uint32), got[:m].view(np.uint32))
+    base = y0 if mode == 1 else np.full((M, N), np.nan, np.float32)
+    assert np.array_equal(part[m:].view(np.uint32), base[m:].view(np.uint32))
+
+
+@pytest.mark.parametrize("GA", [None, 32])
+def test_wave_gemm_special_values(GA):
+    """NaN and infinite scales stay in their own rows and columns: a NaN
+    activation scale spoils its token, an infinite weight scale its column,
+    a zero activation scale gives a zero row; everything else is unchanged."""
+    M, K, N, G = 40, 512, 70, 32
+    rng = np.random.default_rng(9)
+    wq, ws = ref.make_weight(rng, N, K, G)
+    xq, dx, xs = orc.quant_act(ref.make_activations(rng, M, K), GA, G)
+    gaa = K if GA is None else GA
+    want = orc.linear(wq, ws, K, G, xq, dx, xs, GA=gaa)
+    dx, ws = dx.copy(), ws.copy()
+    dx[3] = np.nan
+    dx[7] = 0.0
+    ws[11, 5] = (ws[11, 5] & 0xFFFF0000) | 0x7C00  # scale = +inf
+    y = ops.gemm(ops.Q4Tensor.from_numpy(wq, ws, K, G), ops.Acts(dev(xq), dev(dx), dev(xs), gaa, G))
+    got = y.cpu().numpy()
+    assert np.isnan(got[3]).all()
+    rest = np.delete(np.arange(M), [3, 7])
+    cols = np.delete(np.arange(N), 11)
+    assert np.array_equal(got[7, cols], np.zeros(N - 1, np.float32))
+    assert not np.isfinite(got[rest, 11]).any()
+    assert rel_err(got[np.ix_(rest, cols)], want[np.ix_(rest, cols)]) < 1e-5

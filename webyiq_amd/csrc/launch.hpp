@@ -126,6 +126,10 @@ hipError_t launch_gemv_mfma(const LinearArgs& a, const ArgmaxArgs* am, hipStream
 hipError_t launch_gemv_quant_in(const LinearArgs& a, const QuantInArgs& q, hipStream_t s);
 hipError_t launch_lm_head_argmax(const LinearArgs& a, const ArgmaxArgs& am, hipStream_t s);
 hipError_t launch_gemm(const LinearArgs& a, hipStream_t s);
+// few tokens, or per-32 activations: the GEMM with K split between the waves
+// of a workgroup (tiled_us: the fitted cost of the 128-token tiles)
+bool gemm_wave_fits(const LinearArgs& a, double tiled_us);
+hipError_t launch_gemm_wave(const LinearArgs& a, hipStream_t s);
 // Bytes of workspace the GEMM's K-split plan needs for this shape (0: the
 // shape never splits).
 size_t gemm_workspace_bytes(const LinearArgs& a);
