@@ -1,0 +1,31 @@
+"""The quantiser's workgroup-per-token layout at the edges of its dispatch:
+255 and 256 tokens (eight and four waves on rows of one pass), one, three,
+four and eight passes, partial passes, and the first row too long for it
+(K = 16512: one wavefront per token).  Codes, scales and sums bit-exact
+against the CPU oracle."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as orc
+from oracle import reference as ref
+from webyiq_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M,K", [(255, 2048), (256, 2048), (257, 128), (256, 1920), (40, 2176), (33, 6144),
+                                 (20, 8192), (18, 16384), (18, 16512)])
+@pytest.mark.parametrize("GA,G,norm", [(None, 128, True), (None, 32, False), (32, 128, True)])
+def test_quant_layout_edges(M, K, GA, G, norm):
+    print(f"[case] quant M={M} K={K} GA={GA} G={G} norm={norm}", flush=True)
+    rng = np.random.default_rng(M + K)
+    x = ref.make_activations(rng, M, K)
+    x[M // 2] = 0.0
+    nw = rng.normal(1.0, 0.2, size=K).astype(np.float32) if norm else None
+    xq, dx, xs = orc.quant_act(x, GA, G, norm_w=nw, eps=1e-6)
+    a = ops.quant(torch.from_numpy(x).cuda(), norm=None if nw is None else torch.from_numpy(nw).cuda(), eps=1e-6,
+                  GA=GA, G=G)
+    assert np.array_equal(a.xq.cpu().numpy(), xq)
+    assert np.array_equal(a.dx.cpu().numpy().view(np.uint32), dx.view(np.uint32))
+    assert np.array_equal(a.xs.cpu().numpy(), xs)

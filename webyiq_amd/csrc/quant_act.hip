@@ -17,10 +17,19 @@
 // same value, so codes are bit-identical across the kernels below and the
 // fused GEMV quantiser.
 //
-// Two layouts: few tokens -- one workgroup of eight waves per token, wave w
-// taking load w of every pass (latency: 1.0 us less than four waves with
-// the RMSNorm, 0.5 us without); many tokens -- one wavefront per token,
-// four tokens per workgroup, no barriers (throughput).
+// One workgroup of eight waves per token, wave w taking load w of every pass:
+// the serial work of a lane (about ten instructions per element) is what a
+// call of up to a few hundred tokens waits for, and from a thousand on the
+// launch runs at the memory rate.  One wavefront per token, four tokens per
+// workgroup, served 17 tokens and more before: M = 97 8.45 -> 3.47 us
+// (K = 6144) and 4.60 -> 3.09 us (K = 2048 with the RMSNorm), M = 1024
+// 13.2 -> 8.9 and 6.05 -> 5.00 us, M = 4096 31.7 -> 24.8 us (5.1 TB/s) and
+// 12.4 -> 11.6 us, K = 10240 at M = 97 32 -> 4.3 us.  Rows of one pass take
+// four waves from 256 tokens on, two loads each: the norm's exchange and the
+// reductions cost less per element (M = 4096, K = 2048 with the RMSNorm
+// 14.0 us at eight waves, 11.6 at four; M = 97 3.09 and 3.25).  Rows of more
+// than eight passes keep one wavefront per token and re-read their row (L2
+// hits) in each phase.
 #include "common.hpp"
 #include "launch.hpp"
 
@@ -33,7 +42,7 @@ constexpr int kQuantThreads = 256;
 constexpr int kQuantWaves = kQuantThreads / 64;
 constexpr int kPassChunks = 512;   // float4 chunks per 2048-element pass
 constexpr int kSplitMaxPasses = 8; // split layout: K <= 16384
-constexpr int kSplitMaxTokens = 16;
+constexpr int64_t kSplitGridTokens = int64_t(1) << 22;  // 512 threads each: below 2^32 threads per grid
 
 __device__ __forceinline__ float4 normed(float4 v, float r, float4 w) {
     v.x = (v.x * r) * w.x;
@@ -77,13 +86,13 @@ __device__ __forceinline__ void emit(const QuantArgs& a, int64_t t, int c, bool 
     }
 }
 
-// One workgroup of QW = 4 or 8 waves per token; wave w holds loads
-// LPW w .. LPW w + LPW - 1 of every pass (LPW = 8 / QW).  The per-wave
+// One workgroup of QW = 4 or 8 waves per token, rows of at most JM passes;
+// wave w holds loads LPW w .. LPW w + LPW - 1 of every pass (LPW = 8 / QW).  The per-wave
 // RMSNorm subtotals meet in the lane tree's own order: with four waves each
 // holds a pair (c0 + c1, ...) and they meet as (s0 + s1) + (s2 + s3); with
 // eight each holds one chunk and they meet as ((s0 + s1) + (s2 + s3)) +
 // ((s4 + s5) + (s6 + s7)).
-template <bool NORM, bool PER_TOKEN, int GE, int QW>
+template <bool NORM, bool PER_TOKEN, int GE, int QW, int JM>
 __global__ __launch_bounds__(64 * QW) void quant_split_kernel(const float* kx, const float* knw, int kK, int kM,
                                                               QuantArgs a) {
     static_assert(QW == 4 || QW == 8, "waves per token");
@@ -96,15 +105,15 @@ __global__ __launch_bounds__(64 * QW) void quant_split_kernel(const float* kx, c
     const int J = (nchunk + kPassChunks - 1) / kPassChunks;
     const float4* xr = reinterpret_cast<const float4*>(a.x + t * a.K);
     const float4* nw = reinterpret_cast<const float4*>(a.norm_w);
-    __shared__ float sub[kSplitMaxPasses][QW][64];  // per-wave lane subtotals
-    __shared__ float red[kSplitMaxPasses];
+    __shared__ float sub[JM][QW][64];  // per-wave lane subtotals
+    __shared__ float red[JM];
     __shared__ float wred[QW];
     const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
     auto chunk = [&](int j, int i) { return kPassChunks * j + 64 * (LPW * wave + i) + lane; };
 
-    float4 xc[kSplitMaxPasses][LPW], wc[kSplitMaxPasses][LPW];
+    float4 xc[JM][LPW], wc[JM][LPW];
 #pragma unroll
-    for (int j = 0; j < kSplitMaxPasses; ++j)
+    for (int j = 0; j < JM; ++j)
 #pragma unroll
         for (int i = 0; i < LPW; ++i) {
             const int c = chunk(j, i);
@@ -123,12 +132,12 @@ __global__ __launch_bounds__(64 * QW) void quant_split_kernel(const float* kx, c
     float r = 1.0f;
     if (NORM) {
 #pragma unroll
-        for (int j = 0; j < kSplitMaxPasses; ++j)
+        for (int j = 0; j < JM; ++j)
             if (j < J) sub[j][wave][lane] = LPW == 2 ? chunk_ss(xc[j][0]) + chunk_ss(xc[j][LPW - 1]) : chunk_ss(xc[j][0]);
         __syncthreads();
         // wave w completes passes w, w + QW, ...: the lane tree, then the lane tree
 #pragma unroll
-        for (int q = 0; q < (kSplitMaxPasses + QW - 1) / QW; ++q) {
+        for (int q = 0; q < (JM + QW - 1) / QW; ++q) {
             const int j = wave + QW * q;
             if (j < J) {
                 const float* sj = &sub[j][0][lane];
@@ -149,7 +158,7 @@ __global__ __launch_bounds__(64 * QW) void quant_split_kernel(const float* kx, c
     if (PER_TOKEN) {
         float m = 0.0f;
 #pragma unroll
-        for (int j = 0; j < kSplitMaxPasses; ++j)
+        for (int j = 0; j < JM; ++j)
 #pragma unroll
             for (int i = 0; i < LPW; ++i) {
                 const int c = chunk(j, i);
@@ -166,7 +175,7 @@ __global__ __launch_bounds__(64 * QW) void quant_split_kernel(const float* kx, c
     }
     const float rtok = 1.0f / dtok;
 #pragma unroll
-    for (int j = 0; j < kSplitMaxPasses; ++j) {
+    for (int j = 0; j < JM; ++j) {
         if (j >= J) break;
 #pragma unroll
         for (int i = 0; i < LPW; ++i) {
@@ -177,10 +186,9 @@ __global__ __launch_bounds__(64 * QW) void quant_split_kernel(const float* kx, c
     }
 }
 
-// One wavefront per token, 4 tokens per workgroup, no barriers.  JC > 0:
-// rows of at most JC passes stay in registers; JC == 0: longer rows are
+// One wavefront per token, 4 tokens per workgroup, no barriers; the row is
 // re-read (L2 hits) in each phase.
-template <bool NORM, bool PER_TOKEN, int GE, int JC>
+template <bool NORM, bool PER_TOKEN, int GE>
 __global__ __launch_bounds__(kQuantThreads) void quant_wave_kernel(const float* kx, const float* knw, int kK, int kM,
                                                                    QuantArgs a) {
     a.x = kx; a.norm_w = knw; a.K = kK; a.M = kM;  // preloaded (leading arguments)
@@ -194,58 +202,26 @@ __global__ __launch_bounds__(kQuantThreads) void quant_wave_kernel(const float* 
     const float4* nw = reinterpret_cast<const float4*>(a.norm_w);
     const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
     auto chunk = [&](int j, int u) { return kPassChunks * j + 64 * u + lane; };
-
-    constexpr int NC = JC > 0 ? JC : 1;
-    float4 xc[NC][8], wc[NC][8];
-    if (JC > 0) {
-#pragma unroll
-        for (int j = 0; j < NC; ++j)
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int c = chunk(j, u);
-                const bool ok = j < J && c < nchunk;
-                const int cc = ok ? c : 0;  // loads from a valid chunk, no branch
-                const float4 xv = xr[cc];
-                xc[j][u] = ok ? xv : zero4;
-                if (NORM) {
-                    const float4 wv = nw[cc];
-                    wc[j][u] = ok ? wv : zero4;
-                }
-            }
-    }
-    // the outputs and epsilon, in SGPRs once the loads are in flight
     pin_arg(a.eps); pin_arg(a.xq); pin_arg(a.dx); pin_arg(a.xs);
     auto raw = [&](int j, int u) -> float4 {
-        if (JC > 0) return xc[JC > 0 ? j : 0][u];
         const int c = chunk(j, u);
         return c < nchunk ? xr[c] : zero4;
     };
     auto nwt = [&](int j, int u) -> float4 {
-        if (JC > 0) return wc[JC > 0 ? j : 0][u];
         const int c = chunk(j, u);
         return c < nchunk ? nw[c] : zero4;
-    };
-    // f(j) for every pass; constant j (registers) when the row is cached
-    auto for_passes = [&](auto&& f) {
-        if constexpr (JC > 0) {
-#pragma unroll
-            for (int j = 0; j < NC; ++j)
-                if (j < J) f(j);
-        } else {
-            for (int j = 0; j < J; ++j) f(j);
-        }
     };
 
     float r = 1.0f;
     if (NORM) {
         float total = 0.0f;
-        for_passes([&](int j) {
+        for (int j = 0; j < J; ++j) {
             float c[8];
 #pragma unroll
             for (int u = 0; u < 8; ++u) c[u] = chunk_ss(raw(j, u));
             const float p = ((c[0] + c[1]) + (c[2] + c[3])) + ((c[4] + c[5]) + (c[6] + c[7]));
             total = total + wave_sum_tree(p);
-        });
+        }
         r = 1.0f / sqrt_rn(mean_of(total, K) + a.eps);
     }
     auto load = [&](int j, int u) -> float4 { return NORM ? normed(raw(j, u), r, nwt(j, u)) : raw(j, u); };
@@ -253,22 +229,22 @@ __global__ __launch_bounds__(kQuantThreads) void quant_wave_kernel(const float* 
     float dtok = 0.0f;
     if (PER_TOKEN) {
         float m = 0.0f;
-        for_passes([&](int j) {
+        for (int j = 0; j < J; ++j) {
 #pragma unroll
             for (int u = 0; u < 8; ++u)
                 if (chunk(j, u) < nchunk) m = fmaxf(m, absmax4(load(j, u)));
-        });
+        }
         dtok = wave_max(m) / 127.0f;
         if (lane == 0) a.dx[t] = dtok;
     }
     const float rtok = 1.0f / dtok;
-    for_passes([&](int j) {
+    for (int j = 0; j < J; ++j) {
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
             const int c = chunk(j, u);
             emit<PER_TOKEN, GE>(a, t, c, c < nchunk, load(j, u), dtok, rtok, lane);
         }
-    });
+    }
 }
 
 // MTP input stage (mtp_in.wgsl:45-89), one wavefront per (token, half), four
@@ -374,9 +350,11 @@ __global__ __launch_bounds__(kQuantThreads) void mtp_in_kernel(MtpInArgs a) {
 
 // MTP input stage for rows of at most kSplitMaxPasses passes: one workgroup
 // of eight waves per (token, half), wave w holding load w of every pass (the
-// few-token quantiser's split).  The sums of squares meet in the lane tree's
+// quantiser's split; JM as there: M = 333, K = 2048 10.6 -> 7.8 us against
+// loads for eight passes in every row).  The sums of squares meet in the lane tree's
 // order through LDS, as in quant_split_kernel, so the codes are
 // bit-identical to mtp_in_kernel's.
+template <int JM>
 __global__ __launch_bounds__(512) void mtp_in_split_kernel(MtpInArgs a) {
     constexpr int QW = 8;
     pin_arg(a.emb); pin_arg(a.x); pin_arg(a.norm_f); pin_arg(a.norm_e); pin_arg(a.norm_h);
@@ -391,14 +369,14 @@ __global__ __launch_bounds__(512) void mtp_in_split_kernel(MtpInArgs a) {
     const float4* src = reinterpret_cast<const float4*>((hidden ? a.x : a.emb) + m * a.K);
     const float4* w0 = reinterpret_cast<const float4*>(hidden ? a.norm_f : a.norm_e);
     const float4* w1 = reinterpret_cast<const float4*>(a.norm_h);
-    __shared__ float sub[kSplitMaxPasses][QW][64];
-    __shared__ float red[kSplitMaxPasses];
+    __shared__ float sub[JM][QW][64];
+    __shared__ float red[JM];
     const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
     auto chunk = [&](int j) { return kPassChunks * j + 64 * wave + lane; };
 
-    float4 xc[kSplitMaxPasses], wc0[kSplitMaxPasses], wc1[kSplitMaxPasses];
+    float4 xc[JM], wc0[JM], wc1[JM];
 #pragma unroll
-    for (int j = 0; j < kSplitMaxPasses; ++j) {
+    for (int j = 0; j < JM; ++j) {
         const int c = chunk(j);
         const bool ok = j < J && c < nchunk;
         xc[j] = ok ? src[c] : zero4;
@@ -415,7 +393,7 @@ __global__ __launch_bounds__(512) void mtp_in_split_kernel(MtpInArgs a) {
     // 1 / rms of the values vals(j) (mtp_in.wgsl:26-42), the lane tree's order
     auto inv_rms = [&](auto&& vals) {
 #pragma unroll
-        for (int j = 0; j < kSplitMaxPasses; ++j)
+        for (int j = 0; j < JM; ++j)
             if (j < J) sub[j][wave][lane] = chunk_ss(vals(j));
         __syncthreads();
         // wave w completes pass w: the tree over the waves, then over the lanes
@@ -440,7 +418,7 @@ __global__ __launch_bounds__(512) void mtp_in_split_kernel(MtpInArgs a) {
     q.dx = a.dx;
     q.xs = a.xs;
 #pragma unroll
-    for (int j = 0; j < kSplitMaxPasses; ++j) {
+    for (int j = 0; j < JM; ++j) {
         if (j >= J) break;
         const int c = chunk(j);
         const float4 v0 = scale(xc[j], r0, wc0[j]);
@@ -448,27 +426,30 @@ __global__ __launch_bounds__(512) void mtp_in_split_kernel(MtpInArgs a) {
     }
 }
 
+template <bool NORM, bool PT, int GE, int QW, int JM>
+hipError_t launch_split(QuantArgs a, hipStream_t s) {
+    const int64_t M = a.M, nd = PT ? 1 : a.K / 32, ns = a.K / GE;
+    for (int64_t t = 0; t < M; t += kSplitGridTokens) {
+        a.M = M - t < kSplitGridTokens ? M - t : kSplitGridTokens;
+        hipLaunchKernelGGL((quant_split_kernel<NORM, PT, GE, QW, JM>), dim3((unsigned)a.M), dim3(64 * QW), 0, s, a.x,
+                           a.norm_w, (int)a.K, (int)a.M, a);
+        a.x += a.M * a.K;
+        a.xq += a.M * a.K;
+        a.dx += a.M * nd;
+        a.xs += a.M * ns;
+    }
+    return hipGetLastError();
+}
+
 template <bool NORM, bool PT, int GE>
 hipError_t dispatch_rows(const QuantArgs& a, hipStream_t s) {
     const int64_t passes = (a.K + 4 * kPassChunks - 1) / (4 * kPassChunks);
-    if (a.M <= kSplitMaxTokens && passes <= kSplitMaxPasses) {
-#ifndef WQ_QUANT_SPLIT_WAVES
-#define WQ_QUANT_SPLIT_WAVES 8
-#endif
-        hipLaunchKernelGGL((quant_split_kernel<NORM, PT, GE, WQ_QUANT_SPLIT_WAVES>), dim3((unsigned)a.M),
-                           dim3(64 * WQ_QUANT_SPLIT_WAVES), 0, s, a.x, a.norm_w, (int)a.K, (int)a.M, a);
-        return hipGetLastError();
-    }
-    dim3 grid((unsigned)((a.M + kQuantWaves - 1) / kQuantWaves)), block(kQuantThreads);
     if (passes <= 1)
-        hipLaunchKernelGGL((quant_wave_kernel<NORM, PT, GE, 1>), grid, block, 0, s, a.x, a.norm_w, (int)a.K,
-                           (int)a.M, a);
-    else if (passes <= 3)
-        hipLaunchKernelGGL((quant_wave_kernel<NORM, PT, GE, 3>), grid, block, 0, s, a.x, a.norm_w, (int)a.K,
-                           (int)a.M, a);
-    else
-        hipLaunchKernelGGL((quant_wave_kernel<NORM, PT, GE, 0>), grid, block, 0, s, a.x, a.norm_w, (int)a.K,
-                           (int)a.M, a);
+        return a.M < 256 ? launch_split<NORM, PT, GE, 8, 1>(a, s) : launch_split<NORM, PT, GE, 4, 1>(a, s);
+    if (passes <= 3) return launch_split<NORM, PT, GE, 8, 3>(a, s);
+    if (passes <= kSplitMaxPasses) return launch_split<NORM, PT, GE, 8, kSplitMaxPasses>(a, s);
+    hipLaunchKernelGGL((quant_wave_kernel<NORM, PT, GE>), dim3((unsigned)((a.M + kQuantWaves - 1) / kQuantWaves)),
+                       dim3(kQuantThreads), 0, s, a.x, a.norm_w, (int)a.K, (int)a.M, a);
     return hipGetLastError();
 }
 
@@ -490,7 +471,10 @@ hipError_t launch_quant_act(const QuantArgs& a, hipStream_t s) {
 hipError_t launch_mtp_in(const MtpInArgs& a, hipStream_t s) {
     const int64_t passes = (a.K + 4 * kPassChunks - 1) / (4 * kPassChunks);
     if (passes <= kSplitMaxPasses && 2 * a.M <= 65535) {
-        hipLaunchKernelGGL(mtp_in_split_kernel, dim3((unsigned)(2 * a.M)), dim3(512), 0, s, a);
+        const dim3 grid((unsigned)(2 * a.M)), block(512);
+        if (passes <= 1) hipLaunchKernelGGL((mtp_in_split_kernel<1>), grid, block, 0, s, a);
+        else if (passes <= 3) hipLaunchKernelGGL((mtp_in_split_kernel<3>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((mtp_in_split_kernel<kSplitMaxPasses>), grid, block, 0, s, a);
         return hipGetLastError();
     }
     dim3 grid((unsigned)((2 * a.M + kQuantWaves - 1) / kQuantWaves)), block(kQuantThreads);
