@@ -34,7 +34,7 @@ TIMELINE_LIB = os.path.join(HERE, "libwebyiq_q4q8_timeline.so")
 TIMELINE_SOURCE = "gemv_q4q8.hip"
 CXX = os.environ.get("CXX", "g++")
 
-SOURCES = ["capi.hip", "quant_act.hip", "gemv_q4q8.hip", "gemv_mfma.hip", "gemm_q4q8.hip", "gemm_wave.hip", "argmax.hip", "embed.hip",
+SOURCES = ["capi.hip", "quant_act.hip", "gemv_q4q8.hip", "gemv_mfma.hip", "gemm_q4q8.hip", "gemm_q4q8_shared.hip", "gemm_wave.hip", "argmax.hip", "embed.hip",
            "attn_combine.hip"]
 CFLAGS = [
     "--offload-arch=gfx950",

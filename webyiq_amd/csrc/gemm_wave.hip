@@ -425,8 +425,8 @@ Plan pick_plan(const LinearArgs& a) {
 
 // Per-32 activations always; per-token activations when the 128-token tiles
 // would leave most CUs idle: the grid fits one workgroup per CU, or the
-// fitted cost (4 us + tile-steps per CU x 0.18 us, 0.27 us with groups of 32)
-// is below that of the other kernel's best plan, `tiled_us`.  Measured, us,
+// fitted cost (4 us + tile-steps per CU x 0.18 us, 0.25 us with groups of 32)
+// is clearly below that of the other kernel's best plan, `tiled_us`.  Measured, us,
 // here / there: M = 97, K = 2048, N = 3072 5.9 / 10.9, gate/up pairs N = 6144
 // 13.0 / 18.2; M = 200 8.7 / 11.0 and 18.8 / 17.8; M = 333 11.2 / 11.3 and
 // 30.1 / 28.6; groups of 32 at M = 333 13.9 / 21.4 and 40.1 / 58.7.
@@ -434,8 +434,8 @@ bool gemm_wave_fits(const LinearArgs& a, double tiled_us) {
     if (a.GA != a.K) return true;
     const int64_t tiles = tiles_of(a, 2);
     if (tiles <= 256) return true;
-    const double us = 4.0 + (a.G == 32 ? 0.27 : 0.18) * (double)tiles * (double)(a.K / kBK) / 256.0;
-    return us < (a.G == 32 ? 2.0 : 0.9) * tiled_us;
+    const double us = 4.0 + (a.G == 32 ? 0.25 : 0.18) * (double)tiles * (double)(a.K / kBK) / 256.0;
+    return us < 0.9 * tiled_us;
 }
 
 // The group-sum dump (a test hook) runs the plan's waves, and with them its

@@ -126,6 +126,8 @@ hipError_t launch_gemv_mfma(const LinearArgs& a, const ArgmaxArgs* am, hipStream
 hipError_t launch_gemv_quant_in(const LinearArgs& a, const QuantInArgs& q, hipStream_t s);
 hipError_t launch_lm_head_argmax(const LinearArgs& a, const ArgmaxArgs& am, hipStream_t s);
 hipError_t launch_gemm(const LinearArgs& a, hipStream_t s);
+// the 128-token tiles of width bn (64, 128, 192), two workgroups per CU
+hipError_t launch_gemm_shared(const LinearArgs& a, int bn, hipStream_t s);
 // few tokens, or per-32 activations: the GEMM with K split between the waves
 // of a workgroup (tiled_us: the fitted cost of the 128-token tiles)
 bool gemm_wave_fits(const LinearArgs& a, double tiled_us);
