@@ -107,4 +107,5 @@ def check(rc):
 
 
 def call(name, *args):
-    return check(getattr(load(), name)(*args))
+    rc = getattr(_lib or load(), name)(*args)
+    return rc if rc == WQ_OK else check(rc)

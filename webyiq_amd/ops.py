@@ -24,7 +24,6 @@ after the op's kernels on that stream.  torch only provides device memory
 and streams.
 """
 import contextlib
-import ctypes
 from dataclasses import dataclass
 from typing import Optional
 
@@ -62,17 +61,29 @@ def _cuda(t, name):
         raise ValueError(f"{name}: on {t.device}, expected a cuda tensor")
 
 
+def _is(t, dtype, shape, device):
+    """Whether _check(t, .., dtype, shape=shape, device=device) would pass, for
+    plain tensors (the usual case, without forming any message)."""
+    return (type(t) is torch.Tensor and t.dtype is dtype and t.shape == shape and t.device == device
+            and t.is_contiguous())
+
+
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+_CURRENT = contextlib.nullcontext()
 
 
 def _on(stream):
     """Make `stream` current for the op's allocations and launches."""
-    return torch.cuda.stream(stream) if stream is not None else contextlib.nullcontext()
+    return torch.cuda.stream(stream) if stream is not None else _CURRENT
 
 
 def _cur():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """The current stream's handle (the raw one: a torch.cuda.Stream object per
+    call costs more than the launch's argument checks)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 @dataclass
@@ -95,6 +106,11 @@ class Q4Tensor:
         return Q4Tensor(q, s, K, G)
 
     def check(self, name="w"):
+        q, K, G = self.q, self.K, self.G
+        if (type(q) is torch.Tensor and q.dim() == 2 and G > 0 and K % G == 0 and K % 8 == 0
+                and _is(q, torch.int32, (q.shape[0], K // 8), q.device)
+                and _is(self.s, torch.int32, (q.shape[0], K // G), q.device)):
+            return self
         if self.G <= 0 or self.K % self.G or self.K % 8:
             raise ValueError(f"{name}: K = {self.K} is not a multiple of the group {self.G}")
         _check(self.q, f"{name}.q", torch.int32, shape=(self.rows, self.K // 8))
@@ -129,6 +145,13 @@ class Acts:
         return self.xq.shape[1]
 
     def check(self, name="acts"):
+        xq, GA = self.xq, self.GA
+        if type(xq) is torch.Tensor and xq.dim() == 2 and min(self.G, GA) > 0:
+            (M, K), Ge = xq.shape, min(self.G, GA)
+            if (K % GA == 0 and K % Ge == 0 and _is(xq, torch.int8, (M, K), xq.device)
+                    and _is(self.dx, torch.float32, (M, K // GA), xq.device)
+                    and _is(self.xs, torch.int32, (M, K // Ge), xq.device)):
+                return self
         if self.xq.dim() != 2:
             raise ValueError(f"{name}.xq: expected [M, K], got shape {tuple(self.xq.shape)}")
         M, K = self.xq.shape
