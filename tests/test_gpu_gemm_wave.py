@@ -67,6 +67,25 @@ def test_wave_gemm_edges(M, K, N, mode, shift, G, GA):
     assert np.array_equal(part[m:].view(np.uint32), base[m:].view(np.uint32))
 
 
+@pytest.mark.parametrize("m", [0, 1, 32, 33, 96, 129, 130, 200])
+def test_wave_gemm_active_tokens(m):
+    """Device Params number the tiles of the step's m tokens only: rows below
+    min(m, M) are those of the call on m tokens, bit for bit (a row's order of
+    sums does not depend on the others), the rest keep their contents."""
+    M, K, N, G = 130, 512, 1090, 32  # 5 token tiles x 18 or 35 row tiles: no multiple of the XCDs
+    print(f"[case] wave gemm params m={m}", flush=True)
+    rng = np.random.default_rng(4)
+    for mode, rows in ((0, N), (2, 2 * N)):
+        w = ops.Q4Tensor.from_numpy(*ref.make_weight(rng, rows, K, G), K, G)
+        a = ops.Acts(*(dev(v) for v in orc.quant_act(ref.make_activations(rng, M, K), 32, G)), 32, G)
+        full = ops.gemm(w, a, mode=mode).cpu().numpy()
+        y = torch.full((M, N), float("nan"), device="cuda")
+        ops.gemm(w, a, mode=mode, y=y, params=ops.make_params(m=m))
+        got, k = y.cpu().numpy(), min(m, M)
+        assert np.array_equal(got[:k].view(np.uint32), full[:k].view(np.uint32))
+        assert np.isnan(got[k:]).all()
+
+
 @pytest.mark.parametrize("GA", [None, 32])
 def test_wave_gemm_special_values(GA):
     """NaN and infinite scales stay in their own rows and columns: a NaN

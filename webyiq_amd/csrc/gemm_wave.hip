@@ -81,7 +81,7 @@ __global__ __launch_bounds__(64 * W) void wave_gemm_kernel(GemmParams p) {
     const LinearArgs& a = p.a;
     pin_arg(a.wq); pin_arg(a.ws); pin_arg(a.xq); pin_arg(a.dx); pin_arg(a.xs); pin_arg(a.y);
     pin_arg(a.N); pin_arg(a.K); pin_arg(a.M); pin_arg(a.params);
-    pin_arg(p.tilesM); pin_arg(p.NE); pin_arg(p.NG); pin_arg(p.first); pin_arg(p.count); pin_arg(p.wide);
+    pin_arg(p.tilesM); pin_arg(p.tilesN); pin_arg(p.NE); pin_arg(p.NG); pin_arg(p.first); pin_arg(p.count); pin_arg(p.wide);
     if (DUMP) pin_arg(a.acc_dump);
 
     const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5;
@@ -94,14 +94,21 @@ __global__ __launch_bounds__(64 * W) void wave_gemm_kernel(GemmParams p) {
     const int64_t N = a.N;
     const int K = (int)a.K, NG = p.NG, NE = p.NE;
 
-    // XCD-aware tile order: the token tiles of one set of weight rows on one XCD
-    const int tiles = p.count, bid = blockIdx.x;
+    // XCD-aware tile order: the token tiles of one set of weight rows on one
+    // XCD.  Only tiles with tokens of this step are numbered, the workgroups
+    // past them leave: with the token tiles past M interleaved, the working
+    // ones landed on every second or fourth CU of the dispatch order and shared
+    // it (19 tokens of a 128-token chunk, per-32, K = 2048, gate/up pairs
+    // N = 6144 19.5 -> 10.1 us; the whole block's chunk 55 -> 43.6 us).
+    const int tilesM = a.params ? (int)((M + 31) / 32) : p.tilesM;
+    const int64_t left = (int64_t)tilesM * p.tilesN - p.first;
+    const int tiles = left < p.count ? (int)left : p.count, bid = blockIdx.x;
+    if (bid >= tiles) return;  // (uniform: nothing issued yet)
     const int xcd = bid % kXcds, li = bid / kXcds;
     const int per = tiles / kXcds, rem = tiles % kXcds;
     const int lt = (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + li + p.first;
-    const int tile_n = lt / p.tilesM, tile_m = lt - tile_n * p.tilesM;
+    const int tile_n = lt / tilesM, tile_m = lt - tile_n * tilesM;
     const int64_t m0 = (int64_t)tile_m * 32;
-    if (m0 >= M) return;  // a token tile past this step's tokens (uniform: nothing issued yet)
     constexpr int OUTW = MODE == 2 ? 32 : 32 * TN;  // output columns per tile
     const int64_t n0 = (int64_t)tile_n * OUTW;
 
