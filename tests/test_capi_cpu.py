@@ -8,6 +8,7 @@ import re
 import pytest
 
 from webyiq_amd import _lib
+from conftest import gemm_form
 
 L = _lib.load()
 A16 = ctypes.c_void_p(0x10000)  # aligned non-null dummies: validation fails before any use
@@ -84,6 +85,25 @@ def test_gemm_workspace_bytes():
     m512 = wsb(2048, 6144, 128, 512, 6144, 1)               # width 64 split in pairs
     assert m512 == ((4 * 32 * 64 + 255) // 256) * 256 + 4 * 32 * 128 * 64 * 4
     assert wsb(2048, 6144, 64, 1024, 6144, 0) == 0           # unsupported group: no plan
+
+
+@pytest.mark.parametrize("M,K,N,G,mode", [
+    (32, 6144, 2048, 128, 0), (128, 6144, 2048, 128, 1), (256, 6144, 2048, 128, 0), (384, 4096, 2048, 32, 0),
+    (200, 8192, 640, 128, 1), (512, 6144, 2048, 128, 1), (1024, 6144, 2048, 128, 0), (512, 6144, 2048, 32, 0),
+    (512, 4096, 1024, 128, 2), (700, 4096, 1000, 32, 1),
+])
+def test_gemm_workspace_is_used(M, K, N, G, mode):
+    """A workspace is asked for exactly where the call then splits K between
+    workgroup pairs: zero for the calls of few tokens that split it between
+    the waves of a workgroup."""
+    nbytes = L.wq_gemm_workspace_bytes(N, K, G, M, K, mode)
+    kernel, rows, _, split = gemm_form(M, K, N, G, None, mode, workspace=True)
+    assert split == (nbytes > 0)
+    assert not (split and kernel == "waves")
+    if split:  # flag lines, then 128 x rows partial sums per tile
+        tiles = -(-M // 128) * -(-N // (rows // 2 if mode == 2 else rows))
+        assert nbytes == (tiles * 64 + 255) // 256 * 256 + tiles * 128 * rows * 4
+        assert not gemm_form(M, K, N, G, None, mode)[3]  # without a workspace: not split
 
 
 def test_matmul_paths():

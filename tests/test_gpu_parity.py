@@ -20,7 +20,7 @@ import torch
 from oracle import oracle as orc
 from oracle import reference as ref
 from webyiq_amd import ops
-from conftest import rel_err
+from conftest import gemm_form, rel_err
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -369,10 +369,11 @@ SPLIT_CASES = [
     # M, K, N, G, mode: shapes whose plan splits K between workgroup pairs
     (1024, 6144, 2048, 128, 0),   # width 128, 256 workgroups
     (512, 6144, 2048, 128, 1),    # width 64, += residual
-    (256, 6144, 2048, 128, 0),
-    (512, 4096, 1024, 128, 2),    # gate/up pairs (width 128)
-    (384, 4096, 2048, 32, 0),     # per-token group 32
-    (200, 8192, 640, 128, 1),     # ragged token and row tiles, 32 steps per half
+    (512, 4096, 1024, 128, 2),    # gate/up pairs
+    (1000, 8192, 777, 128, 1),    # ragged token and row tiles, 32 steps per half
+    (512, 6144, 2048, 32, 1),     # per-token group 32, width 64
+    (1000, 4608, 2048, 32, 0),    # group 32, width 128, ragged token tiles, 18 steps per half
+    (500, 6144, 1000, 32, 2),     # group 32, gate/up pairs, ragged token and row tiles
 ]
 
 
@@ -392,6 +393,8 @@ def test_gemm_split_k(M, K, N, G, mode):
     a = dev_acts(xq, dx, xs, K, G)
     nws = ops._lib.load().wq_gemm_workspace_bytes(N, K, G, M, K, mode)
     assert nws > 0, "this shape should split"
+    form = gemm_form(M, K, N, G, None, mode, workspace=True)
+    assert form[0] == "tiles" and form[3], form
     wsp = ops.gemm_workspace(N, K, G, M, mode=mode)
     runs = [host(ops.gemm(w, a, mode=mode, y=dev(y0) if mode == 1 else None, workspace=wsp)) for _ in range(3)]
     for r in runs[1:]:

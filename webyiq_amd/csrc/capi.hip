@@ -158,6 +158,22 @@ wq::LinearArgs make_args(const uint32_t* wq, const uint32_t* ws, int64_t N, int6
     return a;
 }
 
+bool gemm_shape_ok(int64_t N, int64_t K, int32_t G, int64_t M, int32_t mode) {
+    return N >= 1 && M >= 1 && K >= 128 && K % 128 == 0 && (G == 32 || G == 128) && mode >= 0 && mode <= 2;
+}
+
+// a product's shape alone, for the GEMM's plan
+wq::LinearArgs shape_args(int64_t N, int64_t K, int32_t G, int64_t M, int32_t GA, int32_t mode) {
+    wq::LinearArgs a{};
+    a.N = N;
+    a.K = K;
+    a.G = G;
+    a.M = M;
+    a.GA = GA;
+    a.mode = mode;
+    return a;
+}
+
 int gemv_impl(const char* fn, void* stream, const uint32_t* wq, const uint32_t* ws, int64_t N,
               int64_t K, int32_t G, const int8_t* xq, const float* dx, const int32_t* xs,
               int64_t M, int32_t GA, int32_t mode, float* y, int32_t* acc) {
@@ -257,15 +273,29 @@ int wq_gemm(void* stream, const uint32_t* wq, const uint32_t* ws, int64_t N, int
 }
 
 size_t wq_gemm_workspace_bytes(int64_t N, int64_t K, int32_t G, int64_t M, int32_t GA, int32_t mode) {
-    if (N < 1 || M < 1 || K < 128 || K % 128 != 0 || (G != 32 && G != 128) || mode < 0 || mode > 2) return 0;
-    wq::LinearArgs a{};
-    a.N = N;
-    a.K = K;
-    a.G = G;
-    a.M = M;
-    a.GA = GA;
-    a.mode = mode;
-    return wq::gemm_workspace_bytes(a);
+    if (!gemm_shape_ok(N, K, G, M, mode)) return 0;
+    return wq::gemm_workspace_bytes(shape_args(N, K, G, M, GA, mode));
+}
+
+// Test hook, host only (in no header; tests/conftest.py binds it): which
+// kernel wq_gemm launches for a shape with a workspace of the given size, into
+// form[4]: wq::GemmForm's kernel, rows, waves and split.
+int wq_gemm_debug_form(int64_t N, int64_t K, int32_t G, int64_t M, int32_t GA, int32_t mode,
+                       size_t workspace_bytes, int32_t* form) {
+    const char* fn = "wq_gemm_debug_form";
+    REQUIRE_PTR(form);
+    if (!gemm_shape_ok(N, K, G, M, mode) || (GA != 32 && (int64_t)GA != K))
+        return fail(WQ_ESHAPE, "%s: no GEMM of N = %lld, K = %lld, G = %d, M = %lld, GA = %d, mode = %d", fn,
+                    (long long)N, (long long)K, G, (long long)M, GA, mode);
+    auto a = shape_args(N, K, G, M, GA, mode);
+    a.workspace = form;  // (only whether there is one counts)
+    a.workspace_bytes = workspace_bytes;
+    const wq::GemmForm f = wq::gemm_form(a);
+    form[0] = f.kernel;
+    form[1] = f.rows;
+    form[2] = f.waves;
+    form[3] = f.split;
+    return ok();
 }
 
 int wq_gemv_debug_acc(void* stream, const uint32_t* wq, const uint32_t* ws, int64_t N, int64_t K,

@@ -110,22 +110,47 @@ hipError_t launch_bn(const LinearArgs& a, const Plan& pl, hipStream_t s) {
     }
 }
 
+// The kernel of a call: the tile plan, and whether the wave-split kernel takes
+// the call instead (the plan then splits nothing).
+struct Choice {
+    Plan tiles;
+    bool wave;
+};
+
+Choice choose(const LinearArgs& a, bool may_split) {
+    Choice c{pick_plan(a, may_split && split_shape(a)), false};
+    c.wave = gemm_wave_fits(a, c.tiles.us);
+    if (c.wave) c.tiles.split = false;
+    return c;
+}
+
+// the same for a call's own workspace
+Choice choose_for(const LinearArgs& a) {
+    const Choice c = choose(a, !a.acc_dump);
+    if (c.tiles.split && !(a.workspace && a.workspace_bytes >= split_bytes(a, c.tiles.bn))) return choose(a, false);
+    return c;
+}
+
 }  // namespace
 
 size_t gemm_workspace_bytes(const LinearArgs& a) {
-    if (!split_shape(a)) return 0;
-    const Plan pl = pick_plan(a, true);
-    return pl.split ? split_bytes(a, pl.bn) : 0;
+    const Choice c = choose(a, true);
+    return c.tiles.split ? split_bytes(a, c.tiles.bn) : 0;
+}
+
+GemmForm gemm_form(const LinearArgs& a) {
+    const Choice c = choose_for(a);
+    if (c.wave) return gemm_wave_form(a);
+    return GemmForm{kFormTiles, c.tiles.bn, 4 * c.tiles.ks, c.tiles.split};
 }
 
 // The group-sum dump (a test hook) runs the tile width the production launch
 // without a workspace picks for the same shape, so the sums it stores are
 // those of the kernel instance that serves the call.
 hipError_t launch_gemm(const LinearArgs& a, hipStream_t s) {
-    Plan pl = pick_plan(a, !a.acc_dump && split_shape(a));
-    if (pl.split && !(a.workspace && a.workspace_bytes >= split_bytes(a, pl.bn))) pl = pick_plan(a, false);
-    if (gemm_wave_fits(a, pl.us)) return launch_gemm_wave(a, s);
-    return a.acc_dump ? launch_bn<true>(a, pl, s) : launch_bn<false>(a, pl, s);
+    const Choice c = choose_for(a);
+    if (c.wave) return launch_gemm_wave(a, s);
+    return a.acc_dump ? launch_bn<true>(a, c.tiles, s) : launch_bn<false>(a, c.tiles, s);
 }
 
 }  // namespace wq

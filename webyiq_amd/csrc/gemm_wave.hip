@@ -445,6 +445,11 @@ bool gemm_wave_fits(const LinearArgs& a, double tiled_us) {
     return us < 0.9 * tiled_us;
 }
 
+GemmForm gemm_wave_form(const LinearArgs& a) {
+    const Plan pl = pick_plan(a);
+    return GemmForm{kFormWaves, 32 * pl.tn, pl.w, false};
+}
+
 // The group-sum dump (a test hook) runs the plan's waves, and with them its
 // fp32 order, on the wide tile; the width does not enter an output's order.
 hipError_t launch_gemm_wave(const LinearArgs& a, hipStream_t s) {

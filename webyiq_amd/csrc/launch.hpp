@@ -135,6 +135,15 @@ hipError_t launch_gemm_wave(const LinearArgs& a, hipStream_t s);
 // Bytes of workspace the GEMM's K-split plan needs for this shape (0: the
 // shape never splits).
 size_t gemm_workspace_bytes(const LinearArgs& a);
+// What launch_gemm runs for these arguments: the kernel, weight rows per tile,
+// waves per workgroup, and whether K is split between workgroup pairs.
+constexpr int kFormTiles = 0, kFormWaves = 1;
+struct GemmForm {
+    int kernel, rows, waves;
+    bool split;
+};
+GemmForm gemm_form(const LinearArgs& a);
+GemmForm gemm_wave_form(const LinearArgs& a);
 hipError_t launch_argmax(const float* logits, int64_t M, int64_t V, const uint32_t* ids,
                          uint32_t* tok_out, hipStream_t s);
 hipError_t launch_fill_zero(void* p, size_t bytes, hipStream_t s);
