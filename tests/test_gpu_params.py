@@ -4,6 +4,8 @@ gemm_q4q8.wgsl:8-13 / attn_combine.wgsl:6-11) on the GPU, through the C ABI.
   * A prefill GEMM recorded for 128 tokens (captured in a HIP graph) covers
     the m tokens the Params buffer holds when it replays: rows 0 .. m-1
     against the oracle, the rows past m untouched (gemm_q4q8.wgsl:69,106).
+    The recorded shapes run the kernel of few tokens; the 128-token tiles are
+    checked eagerly, with one and two wave groups, at every kind of m.
   * A decode layer with the chunk merge, captured once, replayed at three
     positions with only the Params buffer rewritten between replays
     (lib.rs:312-314): each replay equals an eager run of the same layer at
@@ -18,7 +20,7 @@ import torch
 from oracle import oracle as orc
 from oracle import reference as ref
 from webyiq_amd import ops
-from conftest import rel_err
+from conftest import gemm_form, rel_err
 
 pytestmark = pytest.mark.gpu
 
@@ -74,6 +76,40 @@ def test_gemm_chunk_follows_params(K, N, mode):
         if m:
             assert rel_err(got[:m], want[:m]) < 1e-5, f"m={m}"
         assert np.array_equal(got[m:].view(np.uint32), base[m:].view(np.uint32)), f"m={m}: rows past m written"
+
+
+@pytest.mark.parametrize("M,K,N,G,mode,waves", [
+    (128, 512, 6144, 128, 2, 8),    # two wave groups, one token tile (a chunk's gate/up product)
+    (389, 640, 6633, 128, 2, 8),    # two wave groups, 256 rows per tile, four token tiles
+    (900, 384, 3484, 32, 1, 8),     # group 32, two wave groups, eight token tiles
+    (403, 640, 8475, 128, 2, 4),    # one wave group
+    (1290, 384, 4639, 32, 0, 4),    # group 32, one wave group, token tiles in runs of four
+])
+def test_gemm_tiles_follow_params(M, K, N, G, mode, waves):
+    """The 128-token tiles number only the token tiles of the step's m tokens:
+    rows below min(m, M) are those of the call on the full capacity bit for
+    bit, the rows past them keep their contents."""
+    form = gemm_form(M, K, N, G, None, mode)
+    assert form[0] == "tiles" and form[2] == waves and not form[3], form
+    note(f"gemm tile params M={M} K={K} N={N} G={G} mode={mode} form={form}")
+    rng = np.random.default_rng(M + K + N)
+    wq, ws = ref.make_weight(rng, 2 * N if mode == 2 else N, K, G)
+    xq, dx, xs = orc.quant_act(ref.make_activations(rng, M, K), None, G)
+    y0 = rng.normal(size=(M, N)).astype(np.float32)
+    w = ops.Q4Tensor.from_numpy(wq, ws, K, G)
+    a = ops.Acts(dev(xq), dev(dx), dev(xs), K, G)
+    base = dev(y0) if mode == 1 else torch.full((M, N), float("nan"), device="cuda")
+    full = ops.gemm(w, a, mode=mode, y=base.clone())
+    t = np.array([0, 127, 128, M // 2, M - 1]) % M
+    want = orc.linear(wq, ws, K, G, xq[t], dx[t], xs[t], mode=mode, y=y0[t] if mode == 1 else None)
+    assert rel_err(host(full)[t], want) < 1e-5
+    params = ops.make_params(m=M)
+    for m in sorted({0, 1, 127, 128, 129, 256, M // 2, M - 1, M, M + 5}):
+        ops.set_params(params, m=m)
+        y = ops.gemm(w, a, mode=mode, y=base.clone(), params=params)
+        k = min(m, M)
+        assert torch.equal(y[:k].view(torch.int32), full[:k].view(torch.int32)), f"m={m}"
+        assert torch.equal(y[k:].view(torch.int32), base[k:].view(torch.int32)), f"m={m}: rows past m written"
 
 
 def test_decode_layer_positions_from_params():

@@ -105,9 +105,16 @@ __global__ __launch_bounds__(KS * kWaveGroup, KS == 1 ? 2 : 1) void gemm_kernel(
     const int K = (int)a.K;
     const int NG = p.NG;  // groups per row of the weights and of the activations
 
-    // XCD-aware tile order: consecutive tiles (same weight rows) on one XCD
-    const int T = p.tilesM * p.tilesN;
+    // XCD-aware tile order: consecutive tiles (same weight rows) on one XCD.
+    // Only token tiles of this step are numbered, the workgroups past them
+    // leave: with the empty ones interleaved, two working ones met on every
+    // eighth CU while the others stood idle (102 of 1,024 tokens, K = 2048,
+    // gate/up pairs N = 6144: 36.9 -> 28.3 us, group 32 72.5 -> 49.5 us; 512 of
+    // 1,024 tokens 39.3 -> 31.4 and 77.3 -> 53.8 us).
+    const int tilesM = a.params ? (int)((M + BM - 1) / BM) : p.tilesM;
+    const int T = tilesM * p.tilesN;
     int bid = blockIdx.x;
+    if (bid >= (p.split ? 2 * T : T)) return;  // (uniform: nothing issued yet)
     // Split K: workgroups T.. 2T-1 take the second half of the
     // K steps of tile bid - T; with T a multiple of 8 the pair shares an XCD.
     // (Widths up to 128 only: the exchange's registers do not fit beside the
@@ -129,13 +136,12 @@ __global__ __launch_bounds__(KS * kWaveGroup, KS == 1 ? 2 : 1) void gemm_kernel(
     // its L2 holds the activations of 4 token tiles rather than of all of them
     // (M = 4096, K = 2048, gate/up pairs N = 6144: 172.8 -> 165.7 us); others
     // keep every token tile of a row tile together (GM = tilesM)
-    const int GM = K >= 4096 || p.tilesM > 8 ? 4 : p.tilesM;
+    const int GM = K >= 4096 || tilesM > 8 ? 4 : tilesM;
     const int grp = lt / (GM * p.tilesN);
-    const int gm = p.tilesM - grp * GM < GM ? p.tilesM - grp * GM : GM;
+    const int gm = tilesM - grp * GM < GM ? tilesM - grp * GM : GM;
     const int off = lt - grp * GM * p.tilesN;
     const int tile_m = grp * GM + off % gm, tile_n = off / gm;
     const int64_t m0 = (int64_t)tile_m * BM;
-    if (m0 >= M) return;  // a token tile past this step's tokens (uniform: nothing issued yet)
     constexpr int OUTW = MODE == 2 ? BN / 2 : BN;  // output columns per tile
     const int64_t n0 = (int64_t)tile_n * OUTW;
 
