@@ -1,8 +1,9 @@
 """The quantiser's workgroup-per-token layout at the edges of its dispatch:
 255 and 256 tokens (eight and four waves on rows of one pass), one, three,
 four and eight passes, partial passes, and the first row too long for it
-(K = 16512: one wavefront per token).  Codes, scales and sums bit-exact
-against the CPU oracle."""
+(K = 16512: one wavefront per token); short rows of many tokens (one wavefront
+per token, the row in registers).  Codes, scales and sums bit-exact against
+the CPU oracle."""
 import numpy as np
 import pytest
 import torch
@@ -21,6 +22,25 @@ def test_quant_layout_edges(M, K, GA, G, norm):
     print(f"[case] quant M={M} K={K} GA={GA} G={G} norm={norm}", flush=True)
     rng = np.random.default_rng(M + K)
     x = ref.make_activations(rng, M, K)
+    x[M // 2] = 0.0
+    nw = rng.normal(1.0, 0.2, size=K).astype(np.float32) if norm else None
+    xq, dx, xs = orc.quant_act(x, GA, G, norm_w=nw, eps=1e-6)
+    a = ops.quant(torch.from_numpy(x).cuda(), norm=None if nw is None else torch.from_numpy(nw).cuda(), eps=1e-6,
+                  GA=GA, G=G)
+    assert np.array_equal(a.xq.cpu().numpy(), xq)
+    assert np.array_equal(a.dx.cpu().numpy().view(np.uint32), dx.view(np.uint32))
+    assert np.array_equal(a.xs.cpu().numpy(), xs)
+
+
+# both sides of the line where short rows change to one wavefront per token,
+# token counts that leave a workgroup of four tokens unfilled
+@pytest.mark.parametrize("M,K", [(2047, 384), (2049, 128), (2050, 1536), (2051, 1664), (4095, 256), (4097, 1024),
+                                 (4098, 1152), (8191, 128), (8193, 1024)])
+@pytest.mark.parametrize("GA,G,norm", [(None, 128, True), (None, 32, False), (32, 128, True), (32, 32, False)])
+def test_quant_short_rows(M, K, GA, G, norm):
+    print(f"[case] quant short rows M={M} K={K} GA={GA} G={G} norm={norm}", flush=True)
+    rng = np.random.default_rng(M + K)
+    x = rng.normal(size=(M, K)).astype(np.float32)
     x[M // 2] = 0.0
     nw = rng.normal(1.0, 0.2, size=K).astype(np.float32) if norm else None
     xq, dx, xs = orc.quant_act(x, GA, G, norm_w=nw, eps=1e-6)

@@ -27,9 +27,16 @@
 // 12.4 -> 11.6 us, K = 10240 at M = 97 32 -> 4.3 us.  Rows of one pass take
 // four waves from 256 tokens on, two loads each: the norm's exchange and the
 // reductions cost less per element (M = 4096, K = 2048 with the RMSNorm
-// 14.0 us at eight waves, 11.6 at four; M = 97 3.09 and 3.25).  Rows of more
-// than eight passes keep one wavefront per token and re-read their row (L2
-// hits) in each phase.
+// 14.0 us at eight waves, 11.6 at four; M = 97 3.09 and 3.25).
+//
+// Short rows leave most waves of such a workgroup idle, and once thousands of
+// tokens fill the chip their exchange and barriers cost more than the split
+// gives: rows of one pass keep one wavefront per token, four tokens per
+// workgroup, the row in registers, there (wave_rows; K = 128 at 16,384 tokens
+// 15.6 us split, 11.8 so; with the RMSNorm 21.5 and 16.4, K = 1024 23.9 and
+// 19.7; at 4,096 tokens 7.6 and 6.6, 8.4 and 7.5).  Rows of more than eight
+// passes have one wavefront per token too and re-read their row (L2 hits) in
+// each phase.
 #include "common.hpp"
 #include "launch.hpp"
 
@@ -43,6 +50,7 @@ constexpr int kQuantWaves = kQuantThreads / 64;
 constexpr int kPassChunks = 512;   // float4 chunks per 2048-element pass
 constexpr int kSplitMaxPasses = 8; // split layout: K <= 16384
 constexpr int64_t kSplitGridTokens = int64_t(1) << 22;  // 512 threads each: below 2^32 threads per grid
+constexpr int64_t kWaveGridTokens = int64_t(1) << 25;   // 64 threads each
 
 __device__ __forceinline__ float4 normed(float4 v, float r, float4 w) {
     v.x = (v.x * r) * w.x;
@@ -186,9 +194,9 @@ __global__ __launch_bounds__(64 * QW) void quant_split_kernel(const float* kx, c
     }
 }
 
-// One wavefront per token, 4 tokens per workgroup, no barriers; the row is
-// re-read (L2 hits) in each phase.
-template <bool NORM, bool PER_TOKEN, int GE>
+// One wavefront per token, 4 tokens per workgroup, no barriers.  ONE: rows of
+// one pass, in registers; otherwise the row is re-read (L2 hits) in each phase.
+template <bool NORM, bool PER_TOKEN, int GE, bool ONE>
 __global__ __launch_bounds__(kQuantThreads) void quant_wave_kernel(const float* kx, const float* knw, int kK, int kM,
                                                                    QuantArgs a) {
     a.x = kx; a.norm_w = knw; a.K = kK; a.M = kM;  // preloaded (leading arguments)
@@ -197,17 +205,33 @@ __global__ __launch_bounds__(kQuantThreads) void quant_wave_kernel(const float* 
     if (t >= a.M) return;  // whole wavefronts; the kernel has no barrier
     const int K = (int)a.K;
     const int nchunk = K / 4;
-    const int J = (nchunk + kPassChunks - 1) / kPassChunks;
+    const int J = ONE ? 1 : (nchunk + kPassChunks - 1) / kPassChunks;
     const float4* xr = reinterpret_cast<const float4*>(a.x + t * a.K);
     const float4* nw = reinterpret_cast<const float4*>(a.norm_w);
     const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
     auto chunk = [&](int j, int u) { return kPassChunks * j + 64 * u + lane; };
+    float4 xc[ONE ? 8 : 1], wc[ONE ? 8 : 1];
+    if (ONE) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int c = chunk(0, u), cc = c < nchunk ? c : 0;  // loads from a valid chunk, no branch
+            const float4 xv = xr[cc];
+            xc[u] = c < nchunk ? xv : zero4;
+            if (NORM) {
+                const float4 wv = nw[cc];
+                wc[u] = c < nchunk ? wv : zero4;
+            }
+        }
+    }
+    // the outputs and epsilon, in SGPRs once the loads are in flight
     pin_arg(a.eps); pin_arg(a.xq); pin_arg(a.dx); pin_arg(a.xs);
     auto raw = [&](int j, int u) -> float4 {
+        if (ONE) return xc[ONE ? u : 0];
         const int c = chunk(j, u);
         return c < nchunk ? xr[c] : zero4;
     };
     auto nwt = [&](int j, int u) -> float4 {
+        if (ONE) return wc[ONE ? u : 0];
         const int c = chunk(j, u);
         return c < nchunk ? nw[c] : zero4;
     };
@@ -441,16 +465,35 @@ hipError_t launch_split(QuantArgs a, hipStream_t s) {
     return hipGetLastError();
 }
 
+// Short rows of many tokens: where one wavefront per token, the row in
+// registers, was ahead of the split.  Measured, us, this / split, per token
+// with the RMSNorm: K = 512 at 1,024 tokens 4.4 / 4.2, 2,048 5.2 / 5.4, 8,192
+// 10.7 / 12.9; K = 1536 at 4,096 8.3 / 9.2, K = 2048 9.5 / 9.7 and at 8,192
+// 16.9 / 15.7; without it K = 512 at 2,048 4.3 / 4.3, 8,192 8.2 / 9.5, K = 1536
+// 13.0 / 11.6; per 32 with the RMSNorm K = 512 at 4,096 7.0 / 7.0, 8,192 10.4 /
+// 10.8, K = 1536 15.9 / 15.0; per 32 without it the split is never behind.
+template <bool NORM, bool PT>
+bool wave_rows(int64_t M, int64_t K) {
+    return K <= (NORM && PT ? 1536 : 1024) && M >= (NORM && PT ? 2048 : PT ? 4096 : 8192) && M <= kWaveGridTokens;
+}
+
+template <bool NORM, bool PT, int GE, bool ONE>
+hipError_t launch_wave(const QuantArgs& a, hipStream_t s) {
+    hipLaunchKernelGGL((quant_wave_kernel<NORM, PT, GE, ONE>), dim3((unsigned)((a.M + kQuantWaves - 1) / kQuantWaves)),
+                       dim3(kQuantThreads), 0, s, a.x, a.norm_w, (int)a.K, (int)a.M, a);
+    return hipGetLastError();
+}
+
 template <bool NORM, bool PT, int GE>
 hipError_t dispatch_rows(const QuantArgs& a, hipStream_t s) {
     const int64_t passes = (a.K + 4 * kPassChunks - 1) / (4 * kPassChunks);
+    if constexpr (NORM || PT)
+        if (wave_rows<NORM, PT>(a.M, a.K)) return launch_wave<NORM, PT, GE, true>(a, s);
     if (passes <= 1)
         return a.M < 256 ? launch_split<NORM, PT, GE, 8, 1>(a, s) : launch_split<NORM, PT, GE, 4, 1>(a, s);
     if (passes <= 3) return launch_split<NORM, PT, GE, 8, 3>(a, s);
     if (passes <= kSplitMaxPasses) return launch_split<NORM, PT, GE, 8, kSplitMaxPasses>(a, s);
-    hipLaunchKernelGGL((quant_wave_kernel<NORM, PT, GE>), dim3((unsigned)((a.M + kQuantWaves - 1) / kQuantWaves)),
-                       dim3(kQuantThreads), 0, s, a.x, a.norm_w, (int)a.K, (int)a.M, a);
-    return hipGetLastError();
+    return launch_wave<NORM, PT, GE, false>(a, s);
 }
 
 template <bool NORM>
