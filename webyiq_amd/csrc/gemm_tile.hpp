@@ -61,7 +61,11 @@ __global__ __launch_bounds__(KS * kWaveGroup, KS == 1 ? 2 : 1) void gemm_kernel(
     constexpr int RED_SZ = KS == 2 ? kWaveGroup * TM * TN * 16 * 4 : 0;
     constexpr int NWAVES = kThreads / 64;
     constexpr int TR_STRIDE = 36;  // floats per row of a wave's 32 x 32 output transpose (16-byte rows)
-    constexpr int TR_SZ = NWAVES * 32 * TR_STRIDE * 4;
+    // floats of a wave's transpose: gate/up subtiles go in pairs, the second 16
+    // banks on from the first
+    constexpr bool PAIRS = MODE == 2 && TN >= 2;
+    constexpr int TR_SUB = 32 * TR_STRIDE + 16, TR_WAVE = PAIRS ? 2 * TR_SUB : TR_SUB;
+    constexpr int TR_SZ = NWAVES * TR_WAVE * 4;
     constexpr int BODY_SZ = RING_SZ > RED_SZ ? RING_SZ : RED_SZ;
     // + the tile's per-token scales; then (per-token group-128 format) the
     // tile's scale words for the whole K range, loaded once: BN rows of NGP
@@ -787,35 +791,44 @@ __global__ __launch_bounds__(KS * kWaveGroup, KS == 1 ? 2 : 1) void gemm_kernel(
     // epilogue: per-token scale and output mode in registers, then each
     // 32 x 32 subtile goes through a per-wave LDS transpose so that every lane
     // stores 16 consecutive bytes of a row (8 lanes cover a 128-byte row
-    // segment) instead of single words down a column
+    // segment) instead of single words down a column.  In mode 2 a subtile
+    // gives 16 outputs per row, half a segment: two adjacent ones are stored
+    // together, since half lines written one after the other cost the memory
+    // more (gate/up pairs, M = 8192, K = 768, N = 1000 41.9 -> 37.8 us, K = 256
+    // 29.8 -> 27.0, M = 4096, K = 1024, N = 3074 68.2 -> 64.3, M = 4096,
+    // K = 2048, N = 6144 154.1 -> 151.3).
     __syncthreads();  // the ring and the exchange area are free again
-    float* tr = reinterpret_cast<float*>(lds) + (tid >> 6) * (32 * TR_STRIDE);
+    float* tr = reinterpret_cast<float*>(lds) + (tid >> 6) * TR_WAVE;
     const bool vec_ok = (reinterpret_cast<uintptr_t>(a.y) & 15) == 0 && (N & 3) == 0;  // 16-byte rows chunks
-    // a lane's four outputs of a row: 8 lanes cover a row's 32 columns, in
-    // mode 2 4 lanes its 16 gate/up pairs
-    constexpr int LPR = MODE == 2 ? 4 : 8, RPP = 64 / LPR, NP = 32 / RPP;
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
         if (KS == 2 && i != wk) continue;
         float dtok[16];
 #pragma unroll
         for (int r = 0; r < 16; ++r) dtok[r] = dx_tile[arow(i, r)];
+        // subtiles j .. j + n - 1
+        auto store = [&](auto jc, auto nc) __attribute__((always_inline)) {
+            constexpr int j = decltype(jc)::value, n = decltype(nc)::value;
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
+            for (int s = 0; s < n; ++s)
 #pragma unroll
-            for (int r = 0; r < 16; ++r)
-                tr[(8 * (r >> 2) + 4 * h + (r & 3)) * TR_STRIDE + l32] = facc[i][j][r] * dtok[r];
+                for (int r = 0; r < 16; ++r)
+                    tr[s * TR_SUB + (8 * (r >> 2) + 4 * h + (r & 3)) * TR_STRIDE + l32] = facc[i][j + s][r] * dtok[r];
             __builtin_amdgcn_wave_barrier();  // LDS operations of a wave complete in order
-            const int c = 4 * (lane % LPR);
+            // a lane's four outputs of a row: 8 lanes cover a row's 32 columns,
+            // in mode 2 4 lanes the 16 gate/up pairs of a subtile
+            constexpr int LPR = MODE == 2 ? 4 * n : 8, RPP = 64 / LPR, NP = 32 / RPP;
+            const int lc = lane % LPR;
+            const float* own = MODE == 2 ? tr + (lc >> 2) * TR_SUB + 4 * (lc & 3) : tr + 4 * lc;
             // first output column (formed from bcol: the other form of the same
             // value left the 256-wide loop's MFMAs in one clump, 72 -> 76 us
             // at M = 4096, K = 6144, N = 2048)
-            int64_t c0 = n0 + bcol(j) - l32 + c;
-            if (MODE == 2) c0 = n0 + ((bcol(j) - l32) >> 1) + c;
+            int64_t c0 = n0 + bcol(j) - l32 + 4 * lc;
+            if (MODE == 2) c0 = n0 + ((bcol(j) - l32) >> 1) + 4 * lc;
             float4 o[NP], yo4[NP];
 #pragma unroll
             for (int q = 0; q < NP; ++q) {
-                const float* row = tr + (RPP * q + lane / LPR) * TR_STRIDE + c;
+                const float* row = own + (RPP * q + lane / LPR) * TR_STRIDE;
                 o[q] = *reinterpret_cast<const float4*>(row);
                 if (MODE == 2) {
                     const float4 u = *reinterpret_cast<const float4*>(row + 16);
@@ -857,7 +870,12 @@ __global__ __launch_bounds__(KS * kWaveGroup, KS == 1 ? 2 : 1) void gemm_kernel(
                 }
             }
             __builtin_amdgcn_wave_barrier();
-        }
+        };
+        constexpr int JS = PAIRS ? 2 : 1;
+        static_for<0, TN / JS>([&](auto b) __attribute__((always_inline)) {
+            store(std::integral_constant<int, JS * decltype(b)::value>{}, std::integral_constant<int, JS>{});
+        });
+        if constexpr (TN % JS != 0) store(std::integral_constant<int, TN - 1>{}, std::integral_constant<int, 1>{});
     }
 }
 
