@@ -15,7 +15,7 @@ import torch
 from oracle import oracle as orc
 from oracle import reference as ref
 from webyiq_amd import ops
-from conftest import rel_err
+from conftest import gemm_form, rel_err
 
 pytestmark = pytest.mark.gpu
 
@@ -65,6 +65,45 @@ def test_wave_gemm_edges(M, K, N, mode, shift, G, GA):
     assert np.array_equal(part[:m].view(np.uint32), got[:m].view(np.uint32))
     base = y0 if mode == 1 else np.full((M, N), np.nan, np.float32)
     assert np.array_equal(part[m:].view(np.uint32), base[m:].view(np.uint32))
+
+
+def sampled(M):
+    """Every token of the first and the last tile, and some of each between."""
+    return np.unique(np.concatenate([np.arange(min(M, 33)), np.arange(max(0, M - 33), M), np.arange(0, M, 29)]))
+
+
+@pytest.mark.parametrize("M,K,N,G,GA,mode,kernel,waves", [
+    (1050, 128, 2017, 32, 32, 0, "waves", 1),     # one step: one wave per tile
+    (1050, 128, 2600, 128, 32, 1, "waves", 1),
+    (1050, 128, 1050, 32, 32, 2, "waves", 1),
+    (1050, 128, 1950, 128, 32, 2, "waves", 1),
+    (1050, 128, 2000, 32, 32, 1, "waves", 4),     # under the line for mode 1
+    (1050, 384, 4100, 32, 32, 1, "waves", 4),     # old values read late
+    (1050, 256, 4100, 128, 32, 1, "waves", 4),
+    (1050, 128, 4100, 128, None, 0, "tiles", 8),  # one step per token: the 128-token tiles
+    (1050, 128, 4100, 32, None, 1, "tiles", 4),
+])
+def test_short_rows_many_tiles(M, K, N, G, GA, mode, kernel, waves):
+    """Rows of one to three steps under many tiles, ragged in tokens and rows;
+    the group-sum dump gives the same bits."""
+    form = gemm_form(M, K, N, G, GA, mode)
+    assert (form[0], form[2]) == (kernel, waves), form
+    print(f"[case] short rows M={M} K={K} N={N} G={G} GA={GA} mode={mode}", flush=True)
+    rng = np.random.default_rng(M + K + N + mode)
+    wq, ws = ref.make_weight(rng, 2 * N if mode == 2 else N, K, G)
+    gaa = K if GA is None else GA
+    xq, dx, xs = orc.quant_act(ref.make_activations(rng, M, K), GA, G)
+    y0 = rng.normal(size=(M, N)).astype(np.float32) if mode == 1 else None
+    w = ops.Q4Tensor.from_numpy(wq, ws, K, G)
+    a = ops.Acts(dev(xq), dev(dx), dev(xs), gaa, G)
+    got = ops.gemm(w, a, mode=mode, y=None if y0 is None else dev(y0)).cpu().numpy()
+    t = sampled(M)
+    want = orc.linear(wq, ws, K, G, xq[t], dx[t], xs[t], mode=mode, y=None if y0 is None else y0[t], GA=gaa)
+    assert rel_err(got[t], want) < 1e-5
+    assert np.isfinite(got).all()
+    y, acc = ops.group_sums(ops.PATH_PREFILL, w, a, mode=mode, y=None if y0 is None else dev(y0))
+    assert np.array_equal(y.cpu().numpy().view(np.uint32), got.view(np.uint32))
+    assert np.array_equal(acc[dev(t)].cpu().numpy(), orc.group_acc(wq, K, min(G, gaa), xq[t]))
 
 
 @pytest.mark.parametrize("m", [0, 1, 32, 33, 96, 129, 130, 200])

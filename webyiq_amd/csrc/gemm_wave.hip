@@ -67,13 +67,15 @@ struct WaveTile {
     static constexpr int NA = A_SZ / 1024, NB = B_SZ / 1024;  // direct-to-LDS instructions of 1 KiB
 };
 
-template <int TN, int W, int G, bool PT, int MODE, bool DUMP>
+// LATE (mode 1): the outputs' old values are read after the last step instead
+// of before the first (see launch_mode)
+template <int TN, int W, int G, bool PT, int MODE, bool DUMP, bool LATE = false>
 __global__ __launch_bounds__(64 * W) void wave_gemm_kernel(GemmParams p) {
     using T = WaveTile<TN, G, PT>;
     constexpr int NES = T::NES, NGS = T::NGS;
     static_assert(MODE != 2 || TN == 2, "mode 2 pairs a gate and an up subtile");
     static_assert(TN == 1 || TN == 2, "tile");
-    constexpr int RED_SZ = W * TN * 4096;  // the waves' sums
+    constexpr int RED_SZ = W == 1 ? 0 : W * TN * 4096;  // the waves' sums
     constexpr int LDS_SZ = W * T::STAGE > RED_SZ ? W * T::STAGE : RED_SZ;
     static_assert(LDS_SZ <= kLdsBytes, "LDS");
     __shared__ __align__(1024) unsigned char lds[LDS_SZ];
@@ -201,7 +203,7 @@ __global__ __launch_bounds__(64 * W) void wave_gemm_kernel(GemmParams p) {
 #pragma unroll
     for (int q = 0; q < UPW; ++q) {
         if (PT) dtok[q] = a.dx[out_t(q) < M ? out_t(q) : M - 1];
-        if (MODE == 1) yold[q] = out_ok(q) ? a.y[out_at(q)] : 0.0f;
+        if (MODE == 1 && !LATE) yold[q] = out_ok(q) ? a.y[out_at(q)] : 0.0f;
     }
 
     const unsigned char* st = lds + wave * T::STAGE;
@@ -337,15 +339,22 @@ __global__ __launch_bounds__(64 * W) void wave_gemm_kernel(GemmParams p) {
     }
 
     // ---------------- the waves' sums, epilogue ----------------
-    __syncthreads();  // every wave has left its stage
     float* red = reinterpret_cast<float*>(lds);  // [wave][j][r][lane]
     constexpr int WS = TN * 16 * 64;
+    if constexpr (W > 1) {
+        __syncthreads();  // every wave has left its stage
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
+        for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) red[wave * WS + (j * 16 + r) * 64 + lane] = facc[j][r];
-    __syncthreads();
+            for (int r = 0; r < 16; ++r) red[wave * WS + (j * 16 + r) * 64 + lane] = facc[j][r];
+        __syncthreads();
+    }
+    if (MODE == 1 && LATE) {
+#pragma unroll
+        for (int q = 0; q < UPW; ++q) yold[q] = out_ok(q) ? a.y[out_at(q)] : 0.0f;
+    }
     auto total = [&](int j, int r) {  // the waves' sums in wave order
+        if constexpr (W == 1) return facc[j][r];
         const float* q = red + (j * 16 + r) * 64 + lane;
         float v = q[0];
 #pragma unroll
@@ -354,7 +363,7 @@ __global__ __launch_bounds__(64 * W) void wave_gemm_kernel(GemmParams p) {
     };
 #pragma unroll
     for (int q = 0; q < UPW; ++q) {
-        const int unit = wave * UPW + q, r = unit & 15, j = unit >> 4;
+        const int unit = W == 1 ? q : wave * UPW + q, r = unit & 15, j = unit >> 4;
         float v = total(j, r);
         float u = MODE == 2 ? total(1, r) : 0.0f;
         if (PT) {
@@ -366,8 +375,17 @@ __global__ __launch_bounds__(64 * W) void wave_gemm_kernel(GemmParams p) {
     }
 }
 
+// Mode 1 with four waves: early reads of the old values overlap the steps, but
+// their addresses take some 60 registers, and with them a third of the waves
+// of a SIMD.  Per-32 calls of many tiles read them late (us, early / late, 2,048
+// tiles M = 2048, K = 1536, N = 2048 40.7 / 36.3, K = 6144 124 / 120; 24,576
+// tiles M = 8192, K = 256, N = 6144 201 / 166; 1,504 tiles 17.4 / 16.0 and 96 /
+// 95; below, and per token, early ones are ahead: M = 600, K = 768, N = 1000
+// 5.9 / 7.2).  One wave per tile always does.
 template <int TN, int W, int G, bool PT, bool DUMP>
 hipError_t launch_mode(GemmParams gp, hipStream_t s) {
+    constexpr bool MAY = !PT && !DUMP && W <= 4;
+    const bool late = W == 1 || (int64_t)gp.tilesM * gp.tilesN >= 2048;
     // a grid holds fewer than 2^32 threads: larger ones as several launches
     const int64_t tiles = (int64_t)gp.tilesM * gp.tilesN, most = (int64_t(1) << 31) / (64 * W);
     for (int64_t first = 0; first < tiles; first += most) {
@@ -376,7 +394,12 @@ hipError_t launch_mode(GemmParams gp, hipStream_t s) {
         dim3 grid((unsigned)gp.count), block(64 * W);
         switch (gp.a.mode) {
             case 0: hipLaunchKernelGGL((wave_gemm_kernel<TN, W, G, PT, 0, DUMP>), grid, block, 0, s, gp); break;
-            case 1: hipLaunchKernelGGL((wave_gemm_kernel<TN, W, G, PT, 1, DUMP>), grid, block, 0, s, gp); break;
+            case 1:
+                if (MAY && late)
+                    hipLaunchKernelGGL((wave_gemm_kernel<TN, W, G, PT, 1, DUMP, MAY>), grid, block, 0, s, gp);
+                else if constexpr (W > 1)
+                    hipLaunchKernelGGL((wave_gemm_kernel<TN, W, G, PT, 1, DUMP>), grid, block, 0, s, gp);
+                break;
             default:
                 if constexpr (TN == 2)
                     hipLaunchKernelGGL((wave_gemm_kernel<TN, W, G, PT, 2, DUMP>), grid, block, 0, s, gp);
@@ -400,7 +423,10 @@ hipError_t launch_tile(const LinearArgs& a, hipStream_t s) {
     gp.NG = (int)(a.K / a.G);
     auto al = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
     gp.wide = al(a.ws) && al(a.xs) && (pt || al(a.dx));
-    if (pt) return a.G == 128 ? launch_mode<TN, W, 128, true, DUMP>(gp, s) : launch_mode<TN, W, 32, true, DUMP>(gp, s);
+    if (pt) {
+        if constexpr (W == 1) return hipErrorInvalidConfiguration;  // (never planned: per-32 activations only)
+        else return a.G == 128 ? launch_mode<TN, W, 128, true, DUMP>(gp, s) : launch_mode<TN, W, 32, true, DUMP>(gp, s);
+    }
     return a.G == 128 ? launch_mode<TN, W, 128, false, DUMP>(gp, s) : launch_mode<TN, W, 32, false, DUMP>(gp, s);
 }
 
@@ -419,13 +445,21 @@ int64_t tiles_of(const LinearArgs& a, int tn) {
 // 32 the fold outweighs the loads and narrow tiles, whose waves hold fewer
 // registers, stay ahead longer: per-32 at M = 333, K = 4096, N = 2048 (704)
 // 24.0 / 21.7 / 18.3, at M = 512, K = 2048, N = 3072 (1,536) 23.2 / 19.4 / 20.3.
+// A row of one step (K = 128) leaves all waves but one without work; past a few
+// tiles per CU the call waits for their exchange and their place on the CU:
+// per-32 calls run one wave per tile there (us, one / four waves, 512 tiles
+// M = 512, N = 2048 6.8 / 6.0, 1,024 tiles 7.6 / 9.4, 24,576 tiles M = 8192,
+// N = 6144 67 / 114; mode 1 at 1,024 tiles 11.1 / 10.4, 1,824 tiles 14 / 18).
+// One step's sum is the same bits either way.
 struct Plan {
     int tn, w;
 };
 Plan pick_plan(const LinearArgs& a) {
     const bool groups32 = a.G == 32 || a.GA != a.K;
     if (a.mode != 2 && tiles_of(a, 1) <= (groups32 ? 768 : 256)) return Plan{1, 8};
-    return Plan{2, tiles_of(a, 2) <= 256 ? 8 : 4};
+    const int64_t tiles = tiles_of(a, 2);
+    if (a.K == kBK && a.GA != a.K && tiles >= (a.mode == 1 ? 1280 : 1024)) return Plan{2, 1};
+    return Plan{2, tiles <= 256 ? 8 : 4};
 }
 
 }  // namespace
@@ -441,6 +475,10 @@ bool gemm_wave_fits(const LinearArgs& a, double tiled_us) {
     if (a.GA != a.K) return true;
     const int64_t tiles = tiles_of(a, 2);
     if (tiles <= 256) return true;
+    // one step (K = 128) of many tiles: the waves mostly exchange zeros (us, here /
+    // there, gate/up pairs N = 6144 at M = 300, 1,920 tiles, 9.4 / 10.2, M = 1500
+    // 36 / 22, group 32 at M = 8192, mode 0 143 / 51)
+    if (a.K == kBK && tiles > 2048) return false;
     const double us = 4.0 + (a.G == 32 ? 0.25 : 0.18) * (double)tiles * (double)(a.K / kBK) / 256.0;
     return us < 0.9 * tiled_us;
 }
@@ -456,6 +494,7 @@ hipError_t launch_gemm_wave(const LinearArgs& a, hipStream_t s) {
     const Plan pl = pick_plan(a);
     if (a.acc_dump) return pl.w == 8 ? launch_tile<2, 8, true>(a, s) : launch_tile<2, 4, true>(a, s);
     if (pl.tn == 1) return launch_tile<1, 8, false>(a, s);
+    if (pl.w == 1) return launch_tile<2, 1, false>(a, s);
     return pl.w == 8 ? launch_tile<2, 8, false>(a, s) : launch_tile<2, 4, false>(a, s);
 }
 
