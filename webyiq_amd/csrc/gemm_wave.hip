@@ -69,7 +69,7 @@ struct WaveTile {
 
 // LATE (mode 1): the outputs' old values are read after the last step instead
 // of before the first (see launch_mode)
-template <int TN, int W, int G, bool PT, int MODE, bool DUMP, bool LATE = false>
+template <int TN, int W, int G, bool PT, int MODE, bool LATE, bool DUMP>
 __global__ __launch_bounds__(64 * W) void wave_gemm_kernel(GemmParams p) {
     using T = WaveTile<TN, G, PT>;
     constexpr int NES = T::NES, NGS = T::NGS;
@@ -393,16 +393,16 @@ hipError_t launch_mode(GemmParams gp, hipStream_t s) {
         gp.count = (int)(tiles - first < most ? tiles - first : most);
         dim3 grid((unsigned)gp.count), block(64 * W);
         switch (gp.a.mode) {
-            case 0: hipLaunchKernelGGL((wave_gemm_kernel<TN, W, G, PT, 0, DUMP>), grid, block, 0, s, gp); break;
+            case 0: hipLaunchKernelGGL((wave_gemm_kernel<TN, W, G, PT, 0, false, DUMP>), grid, block, 0, s, gp); break;
             case 1:
                 if (MAY && late)
-                    hipLaunchKernelGGL((wave_gemm_kernel<TN, W, G, PT, 1, DUMP, MAY>), grid, block, 0, s, gp);
+                    hipLaunchKernelGGL((wave_gemm_kernel<TN, W, G, PT, 1, MAY, DUMP>), grid, block, 0, s, gp);
                 else if constexpr (W > 1)
-                    hipLaunchKernelGGL((wave_gemm_kernel<TN, W, G, PT, 1, DUMP>), grid, block, 0, s, gp);
+                    hipLaunchKernelGGL((wave_gemm_kernel<TN, W, G, PT, 1, false, DUMP>), grid, block, 0, s, gp);
                 break;
             default:
                 if constexpr (TN == 2)
-                    hipLaunchKernelGGL((wave_gemm_kernel<TN, W, G, PT, 2, DUMP>), grid, block, 0, s, gp);
+                    hipLaunchKernelGGL((wave_gemm_kernel<TN, W, G, PT, 2, false, DUMP>), grid, block, 0, s, gp);
                 else
                     return hipErrorInvalidConfiguration;  // the host pairs mode 2 with two columns
                 break;
