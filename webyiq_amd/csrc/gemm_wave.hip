@@ -385,6 +385,9 @@ __global__ __launch_bounds__(64 * W) void wave_gemm_kernel(GemmParams p) {
 template <int TN, int W, int G, bool PT, bool DUMP>
 hipError_t launch_mode(GemmParams gp, hipStream_t s) {
     constexpr bool MAY = !PT && !DUMP && W <= 4;
+    // groups of 32 keep narrow tiles up to 768 of them and run wide ones with
+    // eight waves up to 256 only, that is in mode 2 alone
+    constexpr bool PAIRS_ONLY = TN == 2 && W == 8 && !DUMP && (G == 32 || !PT);
     const bool late = W == 1 || (int64_t)gp.tilesM * gp.tilesN >= 2048;
     // a grid holds fewer than 2^32 threads: larger ones as several launches
     const int64_t tiles = (int64_t)gp.tilesM * gp.tilesN, most = (int64_t(1) << 31) / (64 * W);
@@ -393,9 +396,13 @@ hipError_t launch_mode(GemmParams gp, hipStream_t s) {
         gp.count = (int)(tiles - first < most ? tiles - first : most);
         dim3 grid((unsigned)gp.count), block(64 * W);
         switch (gp.a.mode) {
-            case 0: hipLaunchKernelGGL((wave_gemm_kernel<TN, W, G, PT, 0, false, DUMP>), grid, block, 0, s, gp); break;
+            case 0:
+                if constexpr (PAIRS_ONLY) return hipErrorInvalidConfiguration;
+                else hipLaunchKernelGGL((wave_gemm_kernel<TN, W, G, PT, 0, false, DUMP>), grid, block, 0, s, gp);
+                break;
             case 1:
-                if (MAY && late)
+                if constexpr (PAIRS_ONLY) return hipErrorInvalidConfiguration;
+                else if (MAY && late)
                     hipLaunchKernelGGL((wave_gemm_kernel<TN, W, G, PT, 1, MAY, DUMP>), grid, block, 0, s, gp);
                 else if constexpr (W > 1)
                     hipLaunchKernelGGL((wave_gemm_kernel<TN, W, G, PT, 1, false, DUMP>), grid, block, 0, s, gp);
