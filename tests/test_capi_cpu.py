@@ -89,7 +89,7 @@ def test_gemm_workspace_bytes():
 
 @pytest.mark.parametrize("M,K,N,G,mode", [
     (32, 6144, 2048, 128, 0), (128, 6144, 2048, 128, 1), (256, 6144, 2048, 128, 0), (384, 4096, 2048, 32, 0),
-    (200, 8192, 640, 128, 1), (512, 6144, 2048, 128, 1), (1024, 6144, 2048, 128, 0), (512, 6144, 2048, 32, 0),
+    (200, 8192, 640, 128, 1), (300, 6144, 2048, 128, 0), (512, 6144, 2048, 128, 1), (1024, 6144, 2048, 128, 0), (512, 6144, 2048, 32, 0),
     (512, 4096, 1024, 128, 2), (700, 4096, 1000, 32, 1),
 ])
 def test_gemm_workspace_is_used(M, K, N, G, mode):

@@ -8,16 +8,23 @@
 // serves per-token activations; per-32 scales, and calls of few tokens, run
 // the kernel of gemm_wave.hip.
 //
-// MI355X design.  A workgroup of 4 waves (2 along M x 2 along N, one per SIMD)
+// MI355X design.  A group of 4 waves (2 along M x 2 along N, one per SIMD)
 // owns a 128-token x BN-row tile, and each wave a 64 x BN/2 block of 32 x 32
 // subtiles computed with v_mfma_i32_32x32x32_i8.  Every tile of a K step (128
 // codes) travels global -> LDS directly (global_load_lds, no registers): the
-// int8 activations, the packed int4 weights, the scale words.  A ring of 4
-// LDS stages keeps 3 steps in flight; each step ends with one barrier,
-// preceded by a wait for exactly the loads of the next step.  Each wave
-// expands its weight fragments from nibbles to int8 in registers.  Tiles
-// are stored in rows whose 16-byte chunks are XOR-swizzled by the row index,
-// so that the 16-byte fragment reads of consecutive rows hit distinct banks.
+// int8 activations, the packed int4 weights, the scale words.  Two forms keep
+// two waves on each SIMD, so that one's folds run beside the other's products:
+// - two wave groups on one tile, one workgroup per CU: they take alternate K
+//   steps on a ring of 4 LDS stages, the loads of the next two steps in flight
+//   while two are computed, one barrier per round, and add their sums at the
+//   end (gemm_tile.hpp, KS = 2);
+// - one wave group on 2 stages, two workgroups per CU: a step's fragments move
+//   to registers, a barrier, and the loads of the step after next go into the
+//   stage they leave (KS = 1).
+// Each wave expands its weight fragments from nibbles to int8 in registers.
+// Tiles are stored in rows whose 16-byte chunks are XOR-swizzled by the row
+// index, so that the 16-byte fragment reads of consecutive rows hit distinct
+// banks.
 //
 // Folding the exact group sums into fp32 is VALU work per output element per
 // group, as much issue time as the MFMAs themselves.  Group 128, and group 32
@@ -42,18 +49,19 @@ int64_t tiles_of(const LinearArgs& a, int bn) {
 //   ks = 2: rounds of 256 workgroups, each c0 + steps x (ca + cb x width);
 //     split (K across a workgroup pair: widths up to 128, K a multiple of 512
 //     with 32 steps or more, a workspace): half the steps plus ~3 us for the
-//     exchange.  It splits where the unsplit grid leaves CUs idle (M = 512 and
-//     256, K = 6144, N = 2048 at width 64: 18.3 and 17.3 us against 24.5 and
-//     24.1 us unsplit).
+//     exchange.  It splits where the unsplit grid leaves CUs idle (K = 6144,
+//     N = 2048 at width 64: M = 512 20.4 us against 25.2 unsplit, M = 300 17.9
+//     against 24.5).
 //   ks = 1: two workgroups per CU side by side, c0 + steps x (ca + cb x width)
 //     for a pair and for a workgroup alone.
-// With ks = 1 a tile's first loads, min term, barriers and epilogue (about 9 of
-// 21 us at 16 steps) run beside another tile's products: M = 2048, K = 2048,
-// N = 6144 48.2 -> 39.6 us (width 192), M = 4096, N = 6144 in pairs 165.7 ->
-// 157 us at width 128; group 32, whose fold takes most of the time,
-// 123 -> 75.9 and 326 -> 281 us.  With one tile per CU the two wave groups of
-// ks = 2 stay ahead: M = 1024, K = 2048, N = 6144 26.1 against 27.8 us (group
-// 32: 63.8 against 50.3).
+// With ks = 1 a tile's first loads, min term, barriers and epilogue run beside
+// another tile's products.  Measured, us, best width of ks = 2 / ks = 1 (back
+// to back in a graph): M = 2048, K = 2048, N = 6144 44.7 / 40.3 (both 192),
+// M = 4096 in pairs 165 / 144 (192), K = 6144, N = 2048 71.4 (256) / 73.0 (128);
+// group 32, whose fold takes most of the time, 94.6 (128) / 78.0 (192) and, in
+// pairs, 371 / 270.  With one tile per CU the two wave groups of ks = 2 stay
+// ahead at group 128: M = 1024, K = 2048, N = 6144 24.5 / 29.6, group 32 63.4 /
+// 52.2.
 struct Plan {
     int bn, ks;
     bool split;

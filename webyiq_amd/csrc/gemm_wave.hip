@@ -23,8 +23,8 @@
 // of one f32 MFMA in the accumulator layout, rounded once like the product it
 // replaces, and the min term sum_g m[n,g] (dx[t,g] X[t,g]) of two groups out
 // of another: both ran on the VALU with LDS reads per element in the kernel
-// before it (M = 19, K = 6144, N = 2048: 120 -> 10.8 us; M = 1024, K = 2048,
-// N = 6144 in pairs: 223 -> 129 us).
+// before it (M = 19, K = 6144, N = 2048: 120 -> 10.6 us; M = 1024, K = 2048,
+// N = 6144 in pairs: 223 -> 117 us).
 #include "common.hpp"
 #include "gemm_common.hpp"
 #include "launch.hpp"
@@ -447,11 +447,11 @@ int64_t tiles_of(const LinearArgs& a, int tn) {
 // past one workgroup per CU, wider tiles read the activations half as often
 // and four waves leave room for more workgroups on a CU.  Measured, us, 64
 // rows x 8 waves / 64 x 4 / 32 x 8: M = 60, K = 2048, N = 3072 (192 tiles of
-// 32 rows) 5.9 / 6.1 / 4.9, M = 130, N = 2048 (320) 5.7 / 6.0 / 6.4, M = 700,
-// K = 1024, N = 2048 (704 tiles of 64 rows) 8.6 / 7.9 / 10.3; with groups of
+// 32 rows) 6.1 / 6.2 / 5.4, M = 130, N = 2048 (320) 6.3 / 6.4 / 7.1, M = 700,
+// K = 1024, N = 2048 (704 tiles of 64 rows) 9.6 / 8.6 / 10.5; with groups of
 // 32 the fold outweighs the loads and narrow tiles, whose waves hold fewer
 // registers, stay ahead longer: per-32 at M = 333, K = 4096, N = 2048 (704)
-// 24.0 / 21.7 / 18.3, at M = 512, K = 2048, N = 3072 (1,536) 23.2 / 19.4 / 20.3.
+// 25.4 / 23.4 / 20.8, at M = 512, K = 2048, N = 3072 (1,536) 23.9 / 19.6 / 22.0.
 // A row of one step (K = 128) leaves all waves but one without work; past a few
 // tiles per CU the call waits for their exchange and their place on the CU:
 // per-32 calls run one wave per tile there (us, one / four waves, 512 tiles
@@ -473,11 +473,13 @@ Plan pick_plan(const LinearArgs& a) {
 
 // Per-32 activations always; per-token activations when the 128-token tiles
 // would leave most CUs idle: the grid fits one workgroup per CU, or the
-// fitted cost (4 us + tile-steps per CU x 0.18 us, 0.25 us with groups of 32)
-// is clearly below that of the other kernel's best plan, `tiled_us`.  Measured, us,
-// here / there: M = 97, K = 2048, N = 3072 5.9 / 10.9, gate/up pairs N = 6144
-// 13.0 / 18.2; M = 200 8.7 / 11.0 and 18.8 / 17.8; M = 333 11.2 / 11.3 and
-// 30.1 / 28.6; groups of 32 at M = 333 13.9 / 21.4 and 40.1 / 58.7.
+// fitted cost (4 us + tile-steps per CU x 0.18 us, 0.197 us from 48 steps on,
+// 0.25 us with groups of 32) is clearly below that of the other kernel's best
+// plan, `tiled_us`.  Measured, us, here / there (its best width; back to back
+// in a graph): K = 2048, N = 3072 at M = 97 6.4 / 11.3, M = 200 8.9 / 11.6,
+// M = 333 11.5 / 11.7; gate/up pairs N = 6144 12.0 / 12.4, 18.3 / 17.9 and
+// 26.5 / 23.0; groups of 32 at M = 333 15.3 / 20.4 and 34.7 / 51.0; K = 6144,
+// N = 2048 at M = 256 12.4 / 17.4, M = 300 18.9 / 17.9 (K split in pairs there).
 bool gemm_wave_fits(const LinearArgs& a, double tiled_us) {
     if (a.GA != a.K) return true;
     const int64_t tiles = tiles_of(a, 2);
@@ -486,7 +488,8 @@ bool gemm_wave_fits(const LinearArgs& a, double tiled_us) {
     // there, gate/up pairs N = 6144 at M = 300, 1,920 tiles, 9.4 / 10.2, M = 1500
     // 36 / 22, group 32 at M = 8192, mode 0 143 / 51)
     if (a.K == kBK && tiles > 2048) return false;
-    const double us = 4.0 + (a.G == 32 ? 0.25 : 0.18) * (double)tiles * (double)(a.K / kBK) / 256.0;
+    const int64_t steps = a.K / kBK;
+    const double us = 4.0 + (a.G == 32 ? 0.25 : steps < 48 ? 0.18 : 0.197) * (double)(tiles * steps) / 256.0;
     return us < 0.9 * tiled_us;
 }
 
