@@ -149,7 +149,10 @@ int wq_quant_gemv(void* stream, const float* x, const float* norm_w, float eps,
  * cores (exact products with per-token activations, fp32 sums in hardware
  * order), and calls of few tokens or with per-32 activations split K between
  * the waves of a workgroup and add the parts in one fixed order: the fp32
- * outputs are deterministic and agree with wq_gemv within rel 1e-5.
+ * outputs are deterministic and agree with wq_gemv within rel 1e-5.  The
+ * shape picks the kernel and with it the order of an output's fp32 sums: the
+ * same row in calls of different M (the capacity, with params) may differ in
+ * its last bits.
  * workspace (device, nullable, 256-byte aligned; no counterpart in the
  * reference): when it holds at least wq_gemm_workspace_bytes(...) > 0 bytes
  * for the call's shape, the K steps of each output tile may be split between
