@@ -1,8 +1,9 @@
 """The GEMM with K split between the waves of a workgroup (gemm_wave.hip),
 against the CPU oracle at the edges of its tiles: 32 tokens x 32 or 64 rows,
-4 or 8 waves, fewer K steps than waves and step counts the waves do not share
-evenly, ragged rows and tokens, and scale, sum and dx arrays that are only
-4-byte aligned (the kernel reads their four-word pieces word by word then).
+1, 4 or 8 waves, fewer K steps than waves and step counts the waves do not
+share evenly, ragged rows and tokens, and scale, sum and dx arrays that are
+only 4-byte aligned (the kernel reads their four-word pieces word by word
+then).  Each case names the form it is there for, which the plan has to give.
 
 fp32 outputs within rel 1e-5 (max-norm) of the oracle, the bar of the other
 GEMM tests: the int32 group sums are exact, and the fp32 sums of K / G terms
@@ -30,21 +31,42 @@ def dev(a, shift=0):
 
 FORMATS = [(128, None), (32, None), (32, 32), (128, 32)]
 
+# M, K, N, mode, shift, rows per tile and waves per workgroup, in every format
+EDGES = [
+    (1, 128, 1, 0, 0, 32, 8),        # one step: seven waves without work
+    (33, 1152, 33, 1, 0, 32, 8),     # nine steps over eight waves, one token and one row past a tile
+    (31, 640, 65, 2, 1, 64, 8),      # gate/up pairs, five steps, unaligned arrays
+    (32, 2048, 97, 0, 3, 32, 8),     # unaligned arrays
+]
+# (groups of 32 keep narrow tiles up to 768 of them, and the 128-token tiles
+# take many of the per-token shapes: each format has its own)
+FOUR_WAVES = [
+    (130, 640, 1700, 2, 1, 128, None),   # gate/up pairs, five steps over four waves, unaligned arrays
+    (130, 640, 1700, 2, 1, 32, None),
+    (130, 640, 1700, 2, 1, 32, 32),
+    (130, 640, 1700, 2, 1, 128, 32),
+    (130, 384, 1700, 2, 0, 32, None),    # three steps over four waves
+    (130, 384, 1700, 2, 0, 32, 32),
+    (130, 384, 1700, 2, 0, 128, 32),
+    (520, 1152, 1555, 0, 2, 32, None),   # nine steps, unaligned arrays
+    (520, 1152, 1555, 0, 2, 32, 32),
+    (520, 1152, 1555, 0, 2, 128, 32),
+    (840, 640, 1025, 1, 0, 32, None),    # eight tokens and one row past a tile
+    (840, 640, 1025, 1, 0, 32, 32),
+    (840, 640, 1025, 1, 0, 128, 32),
+    (300, 1024, 2048, 0, 1, 128, None),
+    (700, 1024, 1024, 1, 0, 128, None),
+]
+CASES = [(*c, G, GA) for c in EDGES for G, GA in FORMATS] + [(*c[:5], 64, 4, *c[5:]) for c in FOUR_WAVES]
 
-@pytest.mark.parametrize("G,GA", FORMATS)
-@pytest.mark.parametrize("M,K,N,mode,shift", [
-    (1, 128, 1, 0, 0),        # one step: seven waves without work
-    (33, 1152, 33, 1, 0),     # nine steps over eight waves, one token and one row past a tile
-    (31, 640, 65, 2, 1),      # gate/up pairs, five steps, unaligned arrays
-    (32, 2048, 97, 0, 3),     # unaligned arrays, narrow tiles
-    (300, 512, 2100, 0, 2),   # more than 256 tiles of 64 rows: four waves, unaligned arrays
-    (520, 384, 1025, 1, 0),   # three steps over four waves
-])
-def test_wave_gemm_edges(M, K, N, mode, shift, G, GA):
+
+@pytest.mark.parametrize("M,K,N,mode,shift,rows,waves,G,GA", CASES)
+def test_wave_gemm_edges(M, K, N, mode, shift, rows, waves, G, GA):
+    form = gemm_form(M, K, N, G, GA, mode)
+    assert form == ("waves", rows, waves, False), form
     print(f"[case] wave gemm M={M} K={K} N={N} G={G} GA={GA} mode={mode} shift={shift}", flush=True)
     rng = np.random.default_rng(M + K + N + mode)
-    rows = 2 * N if mode == 2 else N
-    wq, ws = ref.make_weight(rng, rows, K, G)
+    wq, ws = ref.make_weight(rng, 2 * N if mode == 2 else N, K, G)
     x = ref.make_activations(rng, M, K)
     gaa = K if GA is None else GA
     xq, dx, xs = orc.quant_act(x, GA, G)
@@ -109,8 +131,9 @@ def test_short_rows_many_tiles(M, K, N, G, GA, mode, kernel, waves):
 @pytest.mark.parametrize("m", [0, 1, 32, 33, 96, 129, 130, 200])
 def test_wave_gemm_active_tokens(m):
     """Device Params number the tiles of the step's m tokens only: rows below
-    min(m, M) are those of the call on m tokens, bit for bit (a row's order of
-    sums does not depend on the others), the rest keep their contents."""
+    min(m, M) are those of the call on the whole capacity M, bit for bit (M
+    picks the kernel and with it a row's order of sums), the rest keep their
+    contents."""
     M, K, N, G = 130, 512, 1090, 32  # 5 token tiles x 18 or 35 row tiles: no multiple of the XCDs
     print(f"[case] wave gemm params m={m}", flush=True)
     rng = np.random.default_rng(4)
@@ -123,6 +146,58 @@ def test_wave_gemm_active_tokens(m):
         got, k = y.cpu().numpy(), min(m, M)
         assert np.array_equal(got[:k].view(np.uint32), full[:k].view(np.uint32))
         assert np.isnan(got[k:]).all()
+
+
+@pytest.mark.parametrize("M,K,N,G,mode", [
+    (256, 6144, 2048, 128, 0), (384, 4096, 2048, 32, 0), (200, 8192, 640, 128, 1),
+])
+def test_wave_gemm_ignores_workspace(M, K, N, G, mode):
+    """Long rows under too few tokens for pairs of workgroups: these calls ask
+    for no workspace, and leave one that they are given alone."""
+    assert gemm_form(M, K, N, G, None, mode, workspace=True)[0] == "waves"
+    print(f"[case] wave gemm with a workspace M={M} K={K} N={N} G={G} mode={mode}", flush=True)
+    rng = np.random.default_rng(M + K + N)
+    wq, ws = ref.make_weight(rng, N, K, G)
+    xq, dx, xs = orc.quant_act(ref.make_activations(rng, M, K), None, G)
+    y0 = rng.normal(size=(M, N)).astype(np.float32)
+    w = ops.Q4Tensor.from_numpy(wq, ws, K, G)
+    a = ops.Acts(dev(xq), dev(dx), dev(xs), K, G)
+    plain = ops.gemm(w, a, mode=mode, y=dev(y0))
+    wsp = torch.zeros(8 << 20, dtype=torch.uint8, device="cuda")
+    given = ops.gemm(w, a, mode=mode, y=dev(y0), workspace=wsp)
+    assert torch.equal(given.view(torch.int32), plain.view(torch.int32))
+    assert not wsp.any()
+    t = sampled(M)
+    want = orc.linear(wq, ws, K, G, xq[t], dx[t], xs[t], mode=mode, y=y0[t] if mode == 1 else None)
+    assert rel_err(plain.cpu().numpy()[t], want) < 1e-5
+
+
+def test_wave_gemm_beyond_one_grid():
+    """More tiles than a grid of 2^32 threads holds: the call goes out as two
+    launches, the second starting with columns 1024 (2^23 tiles of 64 rows are
+    16 columns of 524,288 token tiles)."""
+    M, K, N, G = (1 << 24) - 1, 256, 1030, 32
+    if torch.cuda.mem_get_info()[0] < 110e9:
+        pytest.skip("the outputs take 69 GB")
+    assert gemm_form(M, K, N, G, 32) == ("waves", 64, 4, False)
+    print(f"[case] wave gemm in two launches M={M} K={K} N={N}", flush=True)
+    rng = np.random.default_rng(6)
+    wq, ws = ref.make_weight(rng, N, K, G)
+    base = orc.quant_act(ref.make_activations(rng, 4099, K), 32, G)  # repeated: row t is row t % 4099
+    n = -(-M // 4099)
+    xq, dx, xs = (dev(v).repeat(n, 1)[:M].contiguous() for v in base)
+    y = torch.empty((M, N), device="cuda")
+    for r in range(0, M, 1 << 22):
+        y[r:r + (1 << 22)] = float("nan")
+    ops.gemm(ops.Q4Tensor.from_numpy(wq, ws, K, G), ops.Acts(xq, dx, xs, 32, G), y=y)
+    want = orc.linear(wq, ws, K, G, *base, GA=32)
+    first = y[:4099].clone()
+    assert rel_err(first.cpu().numpy(), want) < 1e-5
+    for r in range(0, M, 4099 * 1024):  # every row like its copy among the first ones
+        part = y[r:r + 4099 * 1024]
+        k = part.shape[0] // 4099
+        assert (part[:k * 4099].view(k, 4099, N) == first).all()
+        assert torch.equal(part[k * 4099:], first[:part.shape[0] - k * 4099])
 
 
 @pytest.mark.parametrize("GA", [None, 32])

@@ -5,9 +5,9 @@ Bars (stated per test):
   * int8 codes, dx, xs, int32 group sums, argmax tokens: bit-exact;
   * GEMV fp32 outputs of modes 0/1: bit-exact against the oracle, which
     restates the GEMV's fold order;
-  * GEMM fp32 outputs (per-token activations at G = 128 and 32 fold the min
-    term separately on an f16 MFMA; per-32 activations fold one chain per
-    output against the GEMV's chains and tree) and mode 2 (device expf vs
+  * GEMM fp32 outputs (the min term is summed on an MFMA, f16 with per-token
+    activations and f32 with per-32 ones, and the K steps in one to eight
+    chains, against the GEMV's chains and tree) and mode 2 (device expf vs
     libm expf): within rel 1e-5 (max-norm) of the oracle;
   * every fp32 output within rel 1e-3 (max-norm) of the torch fake-quant path.
 """
@@ -265,6 +265,8 @@ def test_cfg3_verify_shapes(M, name, K, N, mode):
 
 # ------------------------------------------------------------------ GEMM ----
 
+# few tokens: all of these run the kernel that splits K between the waves of a
+# workgroup (the 128-token tiles: tests/test_gpu_gemm_shared.py)
 GEMM_CASES = [
     (256, 2048, 512, 128, None, 0),
     (100, 2048, 384, 128, None, 1),   # ragged M tile
@@ -275,12 +277,12 @@ GEMM_CASES = [
     (17, 512, 64, 32, None, 1),
     (48, 1024, 128, 128, 32, 2),
     (1, 128, 16, 128, None, 0),
-    (200, 2048, 320, 128, None, 2),   # mode 2 at width 256
+    (200, 2048, 320, 128, None, 2),
     (129, 1024, 130, 32, None, 0),
-    (300, 6144, 2048, 128, None, 1),  # down-projection shape, tile width 64
-    (64, 4096, 256, 128, None, 2),    # 32 steps: scale words preloaded, gate/up pairs
-    (70, 3072, 192, 128, None, 0),    # 3 min-term blocks over two wave groups
-    (40, 2176, 130, 128, None, 1),    # 17 groups: min-term blocks word by word
+    (300, 6144, 2048, 128, None, 1),  # down-projection shape
+    (64, 4096, 256, 128, None, 2),    # 32 steps, gate/up pairs
+    (70, 3072, 192, 128, None, 0),
+    (40, 2176, 130, 128, None, 1),    # 17 groups
 ]
 
 
@@ -299,9 +301,8 @@ def test_gemm_bit_exact(M, K, N, G, GA, mode):
     y, acc = ops.group_sums(ops.PATH_PREFILL, w, a, mode=mode, y=dev(y0) if mode == 1 else None)
     assert np.array_equal(host(acc), acc_want)
     got = host(y)
-    # f16-MFMA min term (per-token activations), device expf (mode 2), or
-    # (per-32 activations) the GEMM's single fold chain against the GEMV's
-    # chains-and-tree order
+    # the waves' sums against the GEMV's chains-and-tree order; f16 (per-32:
+    # f32) MFMA min term; device expf (mode 2)
     assert rel_err(got, want) < 1e-5
     # the plain entry point (its own tile width) computes the same values
     y2 = host(ops.gemm(w, a, mode=mode, y=dev(y0) if mode == 1 else None))
@@ -310,8 +311,9 @@ def test_gemm_bit_exact(M, K, N, G, GA, mode):
     assert rel_err(got, fq) < 1e-3
 
 
-# tile width the launcher picks for M = 1024 (8 tiles along M): 192, 256, 128,
-# 256 (mode 2), 64; the other formats at width 128
+# tile width the launcher picks for M = 1024 (8 tiles along M): 192, 192, 256,
+# 128, 256 (mode 2), 64, group 32 128; the last runs the kernel that splits K
+# between waves
 WIDE_CASES = [
     (2048, 6144, 128, None, 0),
     (4096, 6144, 128, None, 0),   # tile width 192, min-term blocks reloaded
@@ -350,10 +352,11 @@ def test_gemm_wide_tiles(K, N, G, GA, mode):
 @pytest.mark.parametrize("M", [256, 512, 2048])
 @pytest.mark.parametrize("K,N", [(2048, 6144), (6144, 2048)])
 def test_gemm_prefill_sizes(M, K, N):
-    """The other prefill sizes, whose tile widths and grids differ from
-    M = 1024's (width 128 at M = 512 and 192 at M = 2048 for N = 6144, 64
-    elsewhere; two rounds of workgroups at M = 2048): every row of the first
-    and the last tile and one row of every 8-row group, against the oracle."""
+    """The other prefill sizes, whose kernels, tile widths and grids differ from
+    M = 1024's (N = 6144: width 64, 128 and 192, the last with two workgroups
+    per CU; N = 2048: K split between waves up to M = 512, width 128 at 2,048):
+    every row of the first and the last tile and one row of every 8-row group,
+    against the oracle."""
     note(f"gemm prefill M={M} K={K} N={N}")
     wq, ws, x, xq, dx, xs = setup_linear(K + N + M, M, K, N, 128, None)
     w = ops.Q4Tensor.from_numpy(wq, ws, K, 128)
@@ -409,6 +412,7 @@ def test_gemm_split_k(M, K, N, G, mode):
     def flags_clear():
         return not host(wsp[: 64 * T]).view(np.uint32)[::16].any()
     assert flags_clear(), "flags left set"
+    assert host(wsp[-(-64 * T // 256) * 256:].view(torch.int32).bool().any()), "no partial sums were handed over"
     got = runs[0]
     unsplit = host(ops.gemm(w, a, mode=mode, y=dev(y0) if mode == 1 else None))
     assert rel_err(got, unsplit) < 1e-5
@@ -431,10 +435,9 @@ def test_gemm_split_k(M, K, N, G, mode):
 
 @pytest.mark.parametrize("M,mode,stride", [(2048, 0, 8), (4096, 2, 32)])
 def test_gemm_group32_wide_widths(M, mode, stride):
-    """Per-token activations at group 32 on the widths the launcher picks for
-    long prompts: 192 at M = 2048, N = 6144 (three columns per wave, the
-    columns' fragments read up front) and 256 in mode 2 at M = 4096 (four
-    columns, read column by column).  Every row of the first and the last
+    """Per-token activations at group 32 on the tiles the launcher picks for
+    long prompts, 192 rows and two workgroups per CU, at M = 2048, N = 6144 and
+    in mode 2 at M = 4096.  Every row of the first and the last
     tile and one row per `stride` elsewhere (offset rotating with the tile),
     against the oracle at rel 1e-5."""
     K, N, G = 2048, 6144, 32
@@ -487,7 +490,8 @@ def test_gemm_long_rows_partial_tile_group():
     """K >= 4096 assigns tiles to XCDs in groups of 4 token tiles; M = 640
     has 5 token tiles, so one full group and a partial one.  Sampled tokens
     of every token tile against the oracle."""
-    M, K, N = 640, 4096, 1024
+    M, K, N = 640, 4096, 2500
+    assert gemm_form(M, K, N, 128)[0] == "tiles"
     note(f"gemm long rows M={M} K={K} N={N}")
     wq, ws, x, xq, dx, xs = setup_linear(641, M, K, N, 128, None)
     w = ops.Q4Tensor.from_numpy(wq, ws, K, 128)

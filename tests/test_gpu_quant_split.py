@@ -49,3 +49,22 @@ def test_quant_short_rows(M, K, GA, G, norm):
     assert np.array_equal(a.xq.cpu().numpy(), xq)
     assert np.array_equal(a.dx.cpu().numpy().view(np.uint32), dx.view(np.uint32))
     assert np.array_equal(a.xs.cpu().numpy(), xs)
+
+
+def test_quant_beyond_one_grid():
+    """More tokens than a grid of 512-thread workgroups holds (2^22): the call
+    goes out as two launches."""
+    M, K, cut = (1 << 22) + 37, 128, 1 << 22
+    print(f"[case] quant in two launches M={M} K={K}", flush=True)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(8)
+    x = torch.randn((M, K), generator=g, device="cuda")
+    a = ops.quant(x, GA=32, G=32)
+    for lo, hi in ((0, 64), (cut - 64, cut), (cut, M)):
+        xq, dx, xs = orc.quant_act(x[lo:hi].cpu().numpy(), 32, 32)
+        assert np.array_equal(a.xq[lo:hi].cpu().numpy(), xq)
+        assert np.array_equal(a.dx[lo:hi].cpu().numpy().view(np.uint32), dx.view(np.uint32))
+        assert np.array_equal(a.xs[lo:hi].cpu().numpy(), xs)
+    for lo, hi in ((0, cut), (cut // 2 + 1, M)):  # the rest: like calls of one launch on its parts
+        b = ops.quant(x[lo:hi], GA=32, G=32)
+        assert torch.equal(b.xq, a.xq[lo:hi]) and torch.equal(b.dx, a.dx[lo:hi]) and torch.equal(b.xs, a.xs[lo:hi])
