@@ -115,10 +115,12 @@ __global__ __launch_bounds__(KS * kWaveGroup, KS == 1 ? 2 : 1) void gemm_kernel(
     // eighth CU while the others stood idle (102 of 1,024 tokens, K = 2048,
     // gate/up pairs N = 6144: 36.9 -> 28.3 us, group 32 72.5 -> 49.5 us; 512 of
     // 1,024 tokens 39.3 -> 31.4 and 77.3 -> 53.8 us).
-    const int tilesM = a.params ? (int)((M + BM - 1) / BM) : p.tilesM;
+    int bid = blockIdx.x, tilesM = p.tilesM;
+    if (a.params) {
+        tilesM = (int)((M + BM - 1) / BM);
+        if (bid >= tilesM * p.tilesN * (p.split ? 2 : 1)) return;  // (uniform: nothing issued yet)
+    }
     const int T = tilesM * p.tilesN;
-    int bid = blockIdx.x;
-    if (bid >= (p.split ? 2 * T : T)) return;  // (uniform: nothing issued yet)
     // Split K: workgroups T.. 2T-1 take the second half of the
     // K steps of tile bid - T; with T a multiple of 8 the pair shares an XCD.
     // (Widths up to 128 only: the exchange's registers do not fit beside the
