@@ -1,4 +1,4 @@
-"""Benchmark of the MI355X int4 x int8 path on BASELINE.json's metric:
+"""Benchmark of the MI355X int4 x int8 path:
 "int4 GEMV us + HBM GB/s (M=1, 2048x6144); prefill GEMM int8 TOPS (M=1024)".
 
   python bench.py [--steps K] [--warmup W] [--copies R] [--no-cpu] [--gpus 1]
@@ -31,8 +31,8 @@ Printed JSON line:
               and fraction of the 5.0 POP/s dense int8 MFMA peak as flat
               keys <shape>_us/_TOPS/_frac; the same shapes at M=256 and 512
               under keys with _M256 / _M512; prefill_detail per shape
-  configs     BASELINE configs 2, 3 and 5, the decode layer, the other
-              producers, one GPU's shard shapes, the group-32 format
+  configs     the decode MLP block, the verify shapes, lm_head + argmax, the
+              decode layer, the other producers, one GPU's shard shapes, the group-32 format
   cpu_baseline the reference's torch fake-quant path (oracle/reference.py) on a
               bounded sample of the same workload on this host's cores
 Algorithmic bytes: W = N*K/2, S = 4*N*K/G, x = M*K + 4*M + 4*M*K/G, y = 4*M*N.
@@ -318,7 +318,7 @@ class Gate:
 def main():
     args = parse()
     if args.gpus != 1:
-        print(f"bench.py: this build measures one GPU only (asked for --gpus {args.gpus}); "
+        print(f"bench.py: measures one GPU only (asked for --gpus {args.gpus}); "
               "the path shards along the output rows, but no multi-GPU run is built", file=sys.stderr)
         sys.exit(2)
     import torch
@@ -534,11 +534,10 @@ def bench_timeline(torch, launch_args):
 
 
 def bench_gemm(torch, lib, ops, orc, ref, args):
-    """M=1024 prefill GEMMs (BASELINE configs[3]); TOPS = 2*M*N*K / time."""
+    """M=1024 prefill GEMMs; TOPS = 2*M*N*K / time."""
     res = {}
     P = ctypes.c_void_p
-    # M = 1024 is BASELINE's shape; 256 and 512 (the smallest prefill sizes
-    # the GEMM path serves) are reported beside it under their own keys
+    # M = 1024 is the headline prefill size; 256 and 512 are reported beside it under their own keys
     for M, K, N in ((1024, 2048, 6144), (1024, 6144, 2048), (512, 2048, 6144), (512, 6144, 2048),
                     (256, 2048, 6144), (256, 6144, 2048)):
         rng = np.random.default_rng(args.seed + K + (0 if M == 1024 else M))
@@ -629,8 +628,7 @@ def parity_gate(name, ok, detail=""):
 
 
 def bench_configs(torch, lib, ops, orc):
-    """BASELINE configs 2, 3 and 5 (decode MLP block, M<=8 verify shapes,
-    lm_head + argmax), one GPU's share of them when split over 2-8 GPUs, and
+    """The decode MLP block, the M<=8 verify shapes and lm_head + argmax, one GPU's share of them when split over 2-8 GPUs, and
     the group-32 format on the cfg-1/2/4 shapes:
     us per launch (graph replays over weight copies, so weights stream from
     HBM) and algorithmic GB/s.  Before timing, every cfg-2/3/5 instance and
@@ -970,7 +968,7 @@ def cpu_model():
 
 def cpu_baseline(torch, ref, wq, ws, K, G, x, nbytes, seconds):
     """The reference's CPU torch fake-quant path (tools/reference.py:35-52,
-    restated in oracle/reference.py) on bounded samples of the BASELINE
+    restated in oracle/reference.py) on bounded samples of the
     workloads, on this host's cores: the headline cfg 1 GEMV (about half of
     `seconds`) and, under "configs", cfg 2 (decode MLP chain), cfg 4 (the
     M=1024 prefill products) and cfg 5 (lm_head + argmax, V=151,936), each

@@ -248,7 +248,7 @@ void or_group_acc(const uint32_t* wq, int64_t N, int64_t K, int Ge,
 }
 
 /* Per-group identity of gemv_q4q8.wgsl:6:  sum_i (q s + m)(xq dx) = dx (s A + m X).
- * Canonical fp32 order shared with the kernels (this build's own; the
+ * Canonical fp32 order shared with the kernels (their own; the
  * reference's subgroup reductions cannot be run here):
  *   per token, G = 128:  per pass of 2048 codes (16 groups), eight chains,
  *                        chain i over the groups 16p + 2i, 16p + 2i + 1 that

@@ -151,7 +151,7 @@ def test_quant_half_boundaries():
 
 GEMV_CASES = [
     # M, K, N, G, GA(None = per token), mode
-    (1, 2048, 6144, 128, None, 0),   # BASELINE cfg 1 shape
+    (1, 2048, 6144, 128, None, 0),   # the headline decode shape
     (1, 2048, 2048, 128, None, 1),
     (1, 6144, 2048, 128, None, 1),   # cfg 2 down
     (1, 2048, 6144, 128, None, 2),   # cfg 2 gate_up (2 x 6144 rows)
@@ -228,7 +228,7 @@ def test_gemv_bit_exact(M, K, N, G, GA, mode):
     assert rel_err(got, fq) < 1e-3
 
 
-# MTP speculative verify (BASELINE configs[2]): the 7 linear shapes of one
+# MTP speculative verify: the 7 linear shapes of one
 # 2B-style layer at M = 2, 4, 8 -- q (2048 -> 2048), k and v (2048 -> 512),
 # o (2048 -> 2048, += residual), gate and up (2048 -> 6144, as two plain
 # products and as the fused gate_up pair), down (6144 -> 2048, += residual)
@@ -239,7 +239,7 @@ VERIFY_SHAPES = [("q", 2048, 2048, 0), ("k_v", 2048, 512, 0), ("o", 2048, 2048, 
 @pytest.mark.parametrize("M", [2, 4, 8])
 @pytest.mark.parametrize("name,K,N,mode", VERIFY_SHAPES)
 def test_cfg3_verify_shapes(M, name, K, N, mode):
-    """Every (M, K x N) pair of configs[2] at group 128, per-token int8: int32
+    """Every (M, K x N) pair of the verify step at group 128, per-token int8: int32
     group sums bit-exact, fp32 bit-exact against the oracle (mode 2 within
     rel 1e-5: device expf), within rel 1e-3 of the torch fake-quant path."""
     note(f"cfg3 {name} M={M} K={K} N={N} mode={mode}")
@@ -456,7 +456,7 @@ def test_gemm_group32_wide_widths(M, mode, stride):
 
 @pytest.mark.parametrize("K,N", [(2048, 6144), (6144, 2048)])
 def test_gemm_prefill_production_int32(K, N):
-    """BASELINE configs[3] at the production tile width (the one the
+    """The M = 1024 prefill products at the production tile width (the one the
     launcher picks for M = 1024): the int32 group sums of all 1,024 tokens
     bit-exact against an exact integer reference (one float64 product per
     group, exact for these magnitudes), and the fp32 output of all 1,024

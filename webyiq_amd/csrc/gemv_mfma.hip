@@ -1,5 +1,5 @@
 // Decode GEMV for 3..8 tokens and long outputs (N >= 16384: the lm_head) on
-// int8 MFMA, per-token activations and weight group 128 (the BASELINE format) -- the operator of gemv_q4q8.hip (webyIQ
+// int8 MFMA, per-token activations and weight group 128 -- the operator of gemv_q4q8.hip (webyIQ
 // crates/engine/src/shaders/gemv_q4q8.wgsl:36-131, Builder::gemv
 // graph.rs:190-198; the lm_head + greedy argmax of graph.rs:476-486 with
 // ARGMAX), for the token counts where the dot4 kernel's per-token VALU work

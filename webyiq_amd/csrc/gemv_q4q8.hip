@@ -19,7 +19,7 @@
 // registers (one token, per-token group 128) or go to LDS.
 // The fp32 epilogue folds each (token, row) in a fixed order the CPU oracle
 // restates, so outputs are bit-reproducible (modes 0 and 1) and the fused
-// argmax sees the same logits.  Per-token group-128 (the BASELINE format):
+// argmax sees the same logits.  Per-token group-128:
 // per 2048-code pass of 16 groups, eight chains c = fma(s, A, c);
 // c = fma(m, X, c) over the pairs of groups (2i, 2i + 1), the pairwise tree
 // over the 8 pair values, the pass sums added in order -- for one token in

@@ -20,14 +20,14 @@
 // One workgroup of eight waves per token, wave w taking load w of every pass:
 // the serial work of a lane (about ten instructions per element) is what a
 // call of up to a few hundred tokens waits for, and from a thousand on the
-// launch runs at the memory rate.  One wavefront per token, four tokens per
-// workgroup, served 17 tokens and more before: M = 97 8.45 -> 3.47 us
-// (K = 6144) and 4.60 -> 3.09 us (K = 2048 with the RMSNorm), M = 1024
-// 13.2 -> 8.9 and 6.05 -> 5.00 us, M = 4096 31.7 -> 24.8 us (5.1 TB/s) and
-// 12.4 -> 11.6 us, K = 10240 at M = 97 32 -> 4.3 us.  Rows of one pass take
-// four waves from 256 tokens on, two loads each: the norm's exchange and the
-// reductions cost less per element (M = 4096, K = 2048 with the RMSNorm
-// 14.0 us at eight waves, 11.6 at four; M = 97 3.09 and 3.25).
+// launch runs at the memory rate.  Against one wavefront per token, four
+// tokens per workgroup (back to back in a graph): M = 97 8.2 -> 3.3 us
+// (K = 6144) and 4.6 -> 3.2 us (K = 2048 with the RMSNorm), M = 1024 9.5 -> 6.0
+// and 5.1 -> 4.4 us, M = 4096 26.1 -> 19.9 and 9.5 -> 9.7 us, K = 10240 at
+// M = 97 24.6 -> 4.1 us.  Rows of one pass take four waves from 256 tokens on,
+// two loads each: the norm's exchange and the reductions cost less per element
+// (K = 2048 with the RMSNorm, us, eight waves / four: M = 256 3.29 / 3.44,
+// M = 1024 4.86 / 4.44, M = 4096 12.4 / 9.6).
 //
 // Short rows leave most waves of such a workgroup idle, and once thousands of
 // tokens fill the chip their exchange and barriers cost more than the split
