@@ -11,13 +11,14 @@
 // fills its own LDS stage by direct global -> LDS loads and waits for its own
 // loads only, so the main loop has no barrier: a step's fragments move to
 // registers, the next step's loads are issued into the stage, and the step is
-// computed meanwhile (a second stage per wave was slower: it halves the
-// workgroups that share a CU).  The waves' fp32 sums meet in LDS at the end,
+// computed meanwhile (a second stage per wave halves the workgroups that share
+// a CU, and was slower where several do).  The waves' fp32 sums meet in LDS at the end,
 // added in wave order.
 //
 // Few tokens are bound by the chain of one workgroup (launch, loads, a few
-// steps, the exchange: 3.4 us at one step per wave, about 0.9 us for each
-// further step), many by the fold.  With groups of 32 each output takes a
+// steps, the exchange: back to back in a graph 4.6-5.0 us at one step per wave,
+// 0.7 us for each further step, 1.1 us with per-32 activations), many by the
+// fold.  With groups of 32 each output takes a
 // conversion and an fma per group on the VALU; per-32 activations need the
 // factor dx[t,g] * s[n,g] besides.  That factor, an outer product, comes out
 // of one f32 MFMA in the accumulator layout, rounded once like the product it
